@@ -163,7 +163,31 @@ void mg_plan_free(MgPlan& mg);
 int mg_solve_ex(MgPlan& mg, const Dims& d, int nsolve, int iguess, hipStream_t st);
 
 // ---- consistent projection (ekm_mgt.hip) --------------------------------------
+// separable solver of the grids without cross terms (ekm_sep.hip)
+struct SepPlan {
+  int on = 0;
+  int nx = 0, ny = 0, nk = 0, j0 = 0;  // columns, rows, eigenmodes (rows with an unknown), the first of them
+  int nmode = 0, nmode64 = 0;         // live kx modes; the first nmode64 solve their lines in FP64
+  int nsolve_max = 0;
+  bool per = false;
+  int pin = -1;                       // pinned point of the singular kx = 0 problem
+  int mt = 0;                         // 16-row tiles per workgroup of the products
+  float* af = nullptr;                // eigenvector products, packed in matrix-core operand order
+  float* ab = nullptr;
+  float* fac = nullptr;               // line factors of modes nmode64..nmode-1
+  double* fac64 = nullptr;            // line factors of modes 0..nmode64-1
+  double* base = nullptr;             // kx-independent diagonal [n], then J [n]
+  double* kx2 = nullptr;              // [nmode]
+  double* wb = nullptr;               // w.b of the singular pair of solves
+  unsigned long long* rmax = nullptr; // max|residual| (bits) of every solve, [iteration][nsolve_max]
+};
 struct TightPlan {
+  SepPlan sep;
+  double tol = 0.0;
+  int maxit = 0;
+  const double* cf64 = nullptr;       // finest-level tables inside mem, for the separable solver
+  const unsigned char* spec = nullptr;
+  const double* wnull = nullptr;
   int fp32 = 0, cm = 0, nsolve_max = 0;
   bool cross = false;                 // operator has cross-derivative terms (9-point)
   bool per = false;                   // periodic z ends

@@ -14,6 +14,8 @@
 // mixed-precision form) with alternating zebra-line Gauss-Seidel smoothing
 // (z lines of both parities, then y lines of both parities), full weighting
 // and bilinear prolongation; the coarsest level gets 20 smoothing steps.
+// The FP32 form on a grid without cross terms (every rectilinear grid) is
+// solved by ekm_sep.hip first; these cycles then serve what that leaves.
 // Line smoothing handles the index-space anisotropy of the stretched grids
 // that makes MUDPACK's point relaxation stall.
 //
@@ -33,6 +35,8 @@
 
 #include "ekm_host.h"
 #include "ekm_internal.h"
+#include "ekm_scan.h"
+#include "ekm_sep.h"
 
 namespace {
 
@@ -99,80 +103,6 @@ struct Ws {
 template <typename T>
 __device__ inline T* wbase(const TLev<T>& L, const Ws<T>& W) {
   return L.lds ? W.s : W.g;
-}
-
-// affine map x -> a*x + b; compose(outer, inner) = outer(inner(x))
-template <typename T>
-struct Aff {
-  T a, b;
-};
-template <typename T>
-__device__ inline Aff<T> compose(const Aff<T>& o, const Aff<T>& i) {
-  return Aff<T>{o.a * i.a, o.a * i.b + o.b};
-}
-
-// Cross-lane moves of the wavefront scans.  dpp<CTRL, RM>(old, v): v of the
-// lane that the DPP control CTRL names, or `old` where that lane lies outside
-// the row or the row is masked out by RM (row_shr:n = 0x110+n, row_shl:n =
-// 0x100+n, row_bcast:15 = 0x142, row_bcast:31 = 0x143; 64-bit values move as
-// two 32-bit halves).
-template <int CTRL, int RM, typename T>
-__device__ inline T dpp(T old, T v) {
-  if constexpr (sizeof(T) == 4) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, RM, 0xf, false));
-  } else {
-    const long long o = __double_as_longlong(old), x = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp((int)o, (int)x, CTRL, RM, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(x >> 32), CTRL, RM, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-  }
-}
-template <typename T>
-__device__ inline T rdlane(T v, int l) {
-  if constexpr (sizeof(T) == 4) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-  } else {
-    const long long x = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)x, l), hi = __builtin_amdgcn_readlane((int)(x >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-  }
-}
-template <int CTRL, int RM, typename T>
-__device__ inline Aff<T> dpp_aff(const Aff<T>& v) {
-  return Aff<T>{dpp<CTRL, RM>((T)1, v.a), dpp<CTRL, RM>((T)0, v.b)};
-}
-
-// inclusive scan over the lanes in increasing order: lane i gets
-// map_i o map_{i-1} o ... o map_0 (in-row doubling steps, then the row
-// prefixes carried by row_bcast:15 to rows 1 and 3 and row_bcast:31 to rows
-// 2 and 3)
-template <typename T>
-__device__ inline Aff<T> wave_scan_up(Aff<T> v) {
-  v = compose(v, dpp_aff<0x111, 0xf>(v));
-  v = compose(v, dpp_aff<0x112, 0xf>(v));
-  v = compose(v, dpp_aff<0x114, 0xf>(v));
-  v = compose(v, dpp_aff<0x118, 0xf>(v));
-  v = compose(v, dpp_aff<0x142, 0xa>(v));
-  v = compose(v, dpp_aff<0x143, 0xc>(v));
-  return v;
-}
-
-// inclusive scan in decreasing order: lane i gets map_i o ... o map_63
-// (in-row doubling steps, then the suffix maps of the rows above, read from
-// the first lane of each row)
-template <typename T>
-__device__ inline Aff<T> wave_scan_down(Aff<T> v) {
-  v = compose(v, dpp_aff<0x101, 0xf>(v));
-  v = compose(v, dpp_aff<0x102, 0xf>(v));
-  v = compose(v, dpp_aff<0x104, 0xf>(v));
-  v = compose(v, dpp_aff<0x108, 0xf>(v));
-  const Aff<T> r1{rdlane(v.a, 16), rdlane(v.b, 16)};
-  const Aff<T> r2{rdlane(v.a, 32), rdlane(v.b, 32)};
-  const Aff<T> r3{rdlane(v.a, 48), rdlane(v.b, 48)};
-  const Aff<T> s2 = r3, s1 = compose(r2, r3), s0 = compose(r1, s1);
-  const int row = (threadIdx.x & 63) >> 4;
-  const Aff<T> tail = row == 0 ? s0 : row == 1 ? s1 : row == 2 ? s2 : Aff<T>{(T)1, (T)0};
-  return compose(v, tail);
 }
 
 // Zebra line relaxation of level L.  The Thomas factors of every line are
@@ -879,12 +809,12 @@ __global__ void __launch_bounds__(NT) k_tight_solve(const TDesc<T>* __restrict__
                                                      double* __restrict__ ws64, const double* __restrict__ rhs_tmp,
                                                      double* __restrict__ phi_out, const double* __restrict__ kx2v,
                                                      int* __restrict__ cycles, int* __restrict__ unconv,
-                                                     size_t plane, const double* __restrict__ guessp, int nsolve) {
+                                                     size_t plane, const double* __restrict__ guessp, int nsolve,
+                                                     const unsigned long long* __restrict__ resume) {
   __shared__ double red[NT];
   __shared__ T ylds[3 * kYMaxTasks * 64];
   extern __shared__ __align__(16) unsigned char tight_lds[];
   const TDesc<T>& g = *gp;
-  const double guess = guessp ? *guessp : 0.0;
   // workgroups are dealt to the 8 XCDs round robin: solves 2m and 2m+1 (the
   // two parts of mode m, which read the same per-mode tables) are placed on
   // one XCD so the second reader finds the tables in that XCD's L2.  The grid
@@ -892,6 +822,14 @@ __global__ void __launch_bounds__(NT) k_tight_solve(const TDesc<T>* __restrict__
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int s = 2 * ((slot >> 1) * 8 + xcd) + (slot & 1);
   if (s >= nsolve) return;
+  // after the separable solver's passes: a solve that met the tolerance is
+  // done, the others go on from phi_out with the cycles that are left
+  if (resume && __longlong_as_double((long long)resume[s]) <= gp->tol) {
+    if (threadIdx.x == 0) unconv[s] = 0;
+    return;
+  }
+  const double guess = resume ? 1.0 : guessp ? *guessp : 0.0;
+  const int it0 = resume ? cycles[s] : 0;
   (void)kx2v;  // the wavenumber enters through the per-mode tables
   T* W = ws + (size_t)s * g.ws;
   const Ws<T> Wp{W, reinterpret_cast<T*>(tight_lds)};
@@ -1003,7 +941,7 @@ __global__ void __launch_bounds__(NT) k_tight_solve(const TDesc<T>* __restrict__
       conv = true;
       break;
     }
-    if (it >= g.maxit) break;
+    if (it0 + it >= g.maxit) break;
     // one cycle on the correction equation: the steps of the mode's program
     // in order, one call site of the smoother
     const T* ainv = fac + g.ainv_off;
@@ -1045,7 +983,7 @@ __global__ void __launch_bounds__(NT) k_tight_solve(const TDesc<T>* __restrict__
     po[p] = phi[(i + 1) + ld * (j + 1)] - shift;
   }
   if (threadIdx.x == 0) {
-    cycles[s] = it;
+    cycles[s] = it0 + it;
     unconv[s] = conv ? 0 : 1;
   }
 }
@@ -1513,6 +1451,18 @@ int tight_build_typed(TightPlan& tp, const ekm_params& p, const Dims& d, const H
   EKM_CHECK(hipMemcpy(d_c964, c964.data(), c964.size() * sizeof(double), hipMemcpyHostToDevice));
   tp.ws_elems = g.ws;
   tp.ws64_elems = g.ws64;
+  tp.tol = g.tol;
+  tp.maxit = g.maxit;
+  tp.cf64 = d_cf64;
+  tp.spec = g.lev[ng].spec;
+  tp.wnull = g.wnull;
+  // FP32 cycles without cross terms: the separable solver where it applies
+  // (not on a plane the cycle solves directly)
+  if (sizeof(T) == 4 && !cross && lc < ng) {
+    const SepProblem q{&hl[ng], spec.data() + loff[ng], per, wnull.empty() ? -1 : g.pin, kx2_mode, nmode};
+    const int e = sep_plan_build(tp.sep, q, tp.nsolve_max);
+    if (e != EKM_OK) return e;
+  }
   return EKM_OK;
 }
 
@@ -1536,6 +1486,7 @@ int tight_plan_build(TightPlan& tp, const ekm_params& p, const Dims& d, const Ho
 }
 
 void tight_plan_free(TightPlan& tp) {
+  sep_plan_free(tp.sep);
   if (tp.mem) (void)hipFree(tp.mem);
   if (tp.fac) (void)hipFree(tp.fac);
   if (tp.ws) (void)hipFree(tp.ws);
@@ -1546,6 +1497,13 @@ void tight_plan_free(TightPlan& tp) {
 int tight_solve_ex(TightPlan& tp, MgPlan& mg, const Dims& d, int nsolve, const double* guess, hipStream_t st) {
   if (nsolve <= 0) return EKM_OK;
   if (nsolve > tp.nsolve_max) return EKM_ERR_ARG;
+  const unsigned long long* resume = nullptr;
+  if (tp.sep.on) {
+    const SepBuffers b{tp.cf64, tp.spec, tp.wnull, tp.tol, tp.maxit, mg.rhs, mg.phi, mg.cycles, tp.ws64, (float*)tp.ws};
+    const int e = sep_solve(tp.sep, b, nsolve, guess, st);
+    if (e != EKM_OK) return e;
+    resume = tp.sep.rmax + (size_t)sep_iters(tp.maxit) * tp.sep.nsolve_max;
+  }
   // a multiple of 16 workgroups for the XCD placement of the solve pairs
   const dim3 grid((unsigned)((nsolve + 15) & ~15));
   // workgroup size: tight_block
@@ -1556,7 +1514,7 @@ int tight_solve_ex(TightPlan& tp, MgPlan& mg, const Dims& d, int nsolve, const d
                                   hipFuncAttributeMaxDynamicSharedMemorySize, tp.lds_bytes));            \
     hipLaunchKernelGGL((k_tight_solve<T, CM, NT, X, PER>), grid, dim3(NT), tp.lds_bytes, st, (const TDesc<T>*)tp.mem, \
                        (T*)tp.ws, tp.ws64, (const double*)mg.rhs, mg.phi, (const double*)mg.kx2, mg.cycles, \
-                       mg.cycles + mg.nsolve_max, d.plane, guess, nsolve);                                                          \
+                       mg.cycles + mg.nsolve_max, d.plane, guess, nsolve, resume);                                                          \
   } while (0)
 #define LAUNCH2(T, CM, X)          \
   do {                             \

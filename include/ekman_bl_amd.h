@@ -78,8 +78,10 @@ typedef struct ekm_params {
    * 1 = consistent projection: on the cells the divergence diagnostic covers
    *     (J=2..NY-1, K=2..NZ-1) the Poisson rows are the divergence of the
    *     projection's own face gradient, so J div u after the projection equals
-   *     the solve's residual; solved by FP32 alternating zebra-line V(1,1)
-   *     cycles inside FP64 iterative refinement until max|residual| <= proj_tol.
+   *     the solve's residual; solved by FP64 alternating zebra-line V(1,1)
+   *     cycles until max|residual| <= proj_tol; 2 = the same with FP32 cycles
+   *     inside FP64 residual iterations, where a grid without cross terms
+   *     takes an FP32 separable solve of the whole plane as its cycle.
    *     Periodic z ends (mudpack_bc 0 0) are supported, periodic y ends are
    *     not (EKM_ERR_UNSUPPORTED); with no specified side the kx = 0 solve
    *     returns the solution with phi = 0 at (K = 0, J = NY+1) that satisfies
@@ -124,7 +126,8 @@ typedef struct ekm_diag {
   int time_step;        /* TIME_STEP */
   int rk_step;          /* next RK_STEP to run (1..3) */
   int mg_solves;        /* real Poisson solves in the last projection */
-  int mg_cycles;        /* W(2,1) cycles summed over those solves (reference iparm(17)) */
+  int mg_cycles;        /* W(2,1) cycles summed over those solves (reference iparm(17)); proj_mode 1, 2:
+                         * V(1,1) cycles and separable solves */
   int mg_max_cycles;    /* largest cycle count of a single solve */
   int status;           /* status of the last substep */
   int mg_unconverged;   /* proj_mode 1/2: solves of the last projection that stopped at proj_maxit
