@@ -135,7 +135,15 @@ struct MgLevel {
   int nx = 0, ny = 0;
   int in_lds = 0;                   // level lives in LDS inside the solve kernel
 };
+// the replica's form for grids without cross terms (ekm_mg5.hip)
+struct Mg5Plan {
+  int on = 0;
+  size_t lds = 0;            // bytes of LDS per solve
+  size_t ws = 0;             // doubles per solve in global memory
+  char* mem = nullptr;       // descriptor, cycle programs, coefficient tables
+};
 struct MgPlan {
+  Mg5Plan five;
   int ngrid = 0;
   int nxa = 0, nxb = 0, nyc = 0, nyd = 0;
   int maxcy = 0;

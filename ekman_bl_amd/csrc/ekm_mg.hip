@@ -25,11 +25,14 @@
 // Stencil coefficients are shared by all solves; only c9 carries the
 // wavenumber, through ce = -kx^2 J: c9 = ((ce - s9) + corr9) reproduces
 // MUDPACK's c9 = ce - (c1+c3+c5+c7) plus its corner correction exactly.
+//
+// Grids without cross terms take ekm_mg5.hip, which gives the same iterates.
 #include <cstring>
 #include <vector>
 
 #include "ekm_host.h"
 #include "ekm_internal.h"
+#include "ekm_mg5.h"
 
 namespace {
 
@@ -694,6 +697,19 @@ void kcycle_program(int kcur, std::vector<int>& ops) {
   for (int r = 0; r < ipost; ++r) emit(OP_RELAX, kcur);
 }
 
+// workspace, cycle counts, wavenumbers, right-hand sides and solutions
+int alloc_planes(MgPlan& mg, const Dims& d) {
+  const int nsolve_max = mg.nsolve_max;
+  EKM_CHECK(hipMalloc(&mg.ws, (size_t)nsolve_max * mg.ws_global * sizeof(double)));
+  EKM_CHECK(hipMalloc(&mg.cycles, (size_t)2 * nsolve_max * sizeof(int)));
+  EKM_CHECK(hipMemset(mg.cycles, 0, (size_t)2 * nsolve_max * sizeof(int)));
+  EKM_CHECK(hipMalloc(&mg.kx2, (size_t)nsolve_max * sizeof(double)));
+  EKM_CHECK(hipMalloc(&mg.rhs, (size_t)nsolve_max * d.plane * sizeof(double)));
+  EKM_CHECK(hipMalloc(&mg.phi, (size_t)nsolve_max * d.plane * sizeof(double)));
+  EKM_CHECK(hipMemset(mg.phi, 0, (size_t)nsolve_max * d.plane * sizeof(double)));
+  return EKM_OK;
+}
+
 }  // namespace
 
 // Host side of the plan: level sizes, LDS split, coefficient tables, phase
@@ -721,6 +737,21 @@ int mg_plan_build(MgPlan& mg, const ekm_params& p, const Dims& d, const HostMetr
     mg.lev[k].nx = nx;
     mg.lev[k].ny = ny;
     coef_total += ((size_t)nx * ny * 11 + 7) & ~(size_t)7;  // each level 64-byte aligned
+  }
+  // cycle programs: full multigrid start, then one W cycle at the finest level
+  std::vector<int> ops;
+  for (int k = 1; k <= mg.ngrid - 1; ++k) {
+    kcycle_program(k, ops);
+    ops.push_back((OP_FMGPROL << 8) | k);
+  }
+  mg.nops_fmg = (int)ops.size();
+  kcycle_program(mg.ngrid, ops);
+  mg.nops_w = (int)ops.size() - mg.nops_fmg;
+  if (mg5_applies(hl, mg.ngrid)) {
+    const int st = mg5_plan_build(mg.five, mg, d, hl, ops, lds_budget_doubles);
+    if (st) return st;
+    mg.ws_global = mg.five.ws;
+    return alloc_planes(mg, d);
   }
   // phase tables of the candidate LDS levels: for colour c and row phase r
   // the points i = ist_c[r] (mod 4 steps), j = r+1 (mod 4 steps), packed as
@@ -822,15 +853,6 @@ int mg_plan_build(MgPlan& mg, const ekm_params& p, const Dims& d, const HostMetr
   lo += red;
   mg.ws_lds = lo;
   if (lo > lds_budget_doubles) return EKM_ERR_UNSUPPORTED;
-  // cycle programs: full multigrid start, then one W cycle at the finest level
-  std::vector<int> ops;
-  for (int k = 1; k <= mg.ngrid - 1; ++k) {
-    kcycle_program(k, ops);
-    ops.push_back((OP_FMGPROL << 8) | k);
-  }
-  mg.nops_fmg = (int)ops.size();
-  kcycle_program(mg.ngrid, ops);
-  mg.nops_w = (int)ops.size() - mg.nops_fmg;
   // coefficient tables: c1..c8 interleaved per point ([p][8], one 64-byte
   // record), then s9, corr9 and the Jacobian of each level
   EKM_CHECK(hipMalloc(&mg.coefmem, coef_total * sizeof(double)));
@@ -884,14 +906,7 @@ int mg_plan_build(MgPlan& mg, const ekm_params& p, const Dims& d, const HostMetr
   if (!tab.empty()) std::memcpy(hbuf.data() + desc_bytes, tab.data(), tab.size() * sizeof(int));
   std::memcpy(hbuf.data() + desc_bytes + tab_bytes, ops.data(), ops_bytes);
   EKM_CHECK(hipMemcpy(dmem, hbuf.data(), hbuf.size(), hipMemcpyHostToDevice));
-  EKM_CHECK(hipMalloc(&mg.ws, (size_t)nsolve_max * mg.ws_global * sizeof(double)));
-  EKM_CHECK(hipMalloc(&mg.cycles, (size_t)2 * nsolve_max * sizeof(int)));
-  EKM_CHECK(hipMemset(mg.cycles, 0, (size_t)2 * nsolve_max * sizeof(int)));
-  EKM_CHECK(hipMalloc(&mg.kx2, (size_t)nsolve_max * sizeof(double)));
-  EKM_CHECK(hipMalloc(&mg.rhs, (size_t)nsolve_max * d.plane * sizeof(double)));
-  EKM_CHECK(hipMalloc(&mg.phi, (size_t)nsolve_max * d.plane * sizeof(double)));
-  EKM_CHECK(hipMemset(mg.phi, 0, (size_t)nsolve_max * d.plane * sizeof(double)));
-  return EKM_OK;
+  return alloc_planes(mg, d);
 }
 
 void mg_plan_free(MgPlan& mg) {
@@ -900,6 +915,8 @@ void mg_plan_free(MgPlan& mg) {
     if (q) (void)hipFree(q);
   if (mg.cycles) (void)hipFree(mg.cycles);
   if (mg.desc) (void)hipFree(mg.desc);
+  if (mg.five.mem) (void)hipFree(mg.five.mem);
+  mg.five = Mg5Plan();
   mg.desc = nullptr;
   mg.ws = mg.coefmem = mg.kx2 = mg.rhs = mg.phi = nullptr;
   mg.cycles = nullptr;
@@ -908,6 +925,7 @@ void mg_plan_free(MgPlan& mg) {
 int mg_solve_ex(MgPlan& mg, const Dims& d, int nsolve, int iguess, hipStream_t st) {
   if (nsolve <= 0) return EKM_OK;
   if (nsolve > mg.nsolve_max) return EKM_ERR_ARG;
+  if (mg.five.on) return mg5_solve(mg, d, nsolve, iguess, st);
   size_t lds = mg.ws_lds * sizeof(double);
   hipLaunchKernelGGL(k_mg_solve, dim3(nsolve), dim3(mg.block), lds, st, (const MgDev*)mg.desc, mg.ws,
                      (const double*)mg.rhs, mg.phi, (const double*)mg.kx2, mg.cycles, d.plane, iguess);
