@@ -373,7 +373,8 @@ __global__ void __launch_bounds__(kBlock) k_flux_accum(Dims d, Metrics M, Ranges
   double kw[R + 1];
 #pragma unroll
   for (int i = 0; i <= R; ++i) {
-    const int m = min(lanep + GW * i, M2);
+    // (modes above NKX stay out of CF and CR: no transform reads them)
+    const int m = min(lanep + GW * i, nkx);
     cf[i] = CF[f0 + m];
     cr[i] = CR[f0 + m];
     w2[i] = tw2[m];
@@ -382,9 +383,9 @@ __global__ void __launch_bounds__(kBlock) k_flux_accum(Dims d, Metrics M, Ranges
 #pragma unroll
   for (int i = 0; i <= R; ++i) {
     const int m = lanep + GW * i;
-    if (m > M2) break;
-    double2 X[2] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
-    if (m <= nkx) {
+    if (m > nkx) break;
+    double2 X[2];
+    {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const double2* Zt = t == 0 ? Zx : Zy;

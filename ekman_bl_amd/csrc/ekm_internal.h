@@ -48,6 +48,22 @@ __host__ __device__ inline size_t mi(const Dims& d, int k, int j) {
   return (size_t)k + (size_t)d.NZ3 * (size_t)j;
 }
 
+// Fourier kernels visit the modes 0..NKX only: the inverse transform reads no
+// other mode and the forward transform writes zeros there, so the third of a
+// field above NKX never reaches a physical value.  kept_mode: mode m of the
+// point at plane index r = k + NZ2 j of this thread (one per kept mode and
+// point), q its element; false past the end.
+__host__ inline size_t kept_modes(const Dims& d) { return (size_t)(d.NKX + 1) * d.plane; }
+__device__ inline bool kept_mode(const Dims& d, int& m, int& k, int& j, size_t& q) {
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x, nm = (unsigned)d.NKX + 1u;
+  const unsigned r = t / nm;
+  m = (int)(t - r * nm);
+  j = (int)(r / (unsigned)d.NZ2);
+  k = (int)(r - (unsigned)j * (unsigned)d.NZ2);
+  q = (size_t)m + (size_t)d.NXC * r;
+  return r < (unsigned)d.plane;
+}
+
 // Index ranges of INIT_DUCT (src/duct.F90:7-232).
 struct Ranges {
   int js, je, zs, ze;

@@ -38,13 +38,9 @@ __device__ inline bool in(int v, int lo, int hi) { return v >= lo && v <= hi; }
 // explicit Fourier-space RHS (src/duct.F90:298-632)
 // ---------------------------------------------------------------------------
 __global__ void k_rhs_fourier(Dims d, Metrics M, RhsArgs a) {
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  int m = (int)(t % d.NXC);
-  size_t r = t / d.NXC;
-  int k = (int)(r % d.NZ2), j = (int)(r / d.NZ2);
-  size_t q = t;
+  int m, k, j;
+  size_t q;
+  if (!kept_mode(d, m, k, j, q)) return;
   const size_t dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
   const double temp3 = a.ss->temp3, temp4 = a.ss->temp4;
   if (in(j, a.rv.js, a.rv.je) && in(k, a.rv.zs, a.rv.ze)) {
@@ -824,14 +820,16 @@ __global__ void k_cfl(Dims d, Metrics M, Ranges r, const double* __restrict__ U1
 __global__ void k_faces(Dims d, Metrics M, Ranges r, const double2* __restrict__ CU2,
                         const double2* __restrict__ CU3, double2* __restrict__ F2,
                         double2* __restrict__ F3) {
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  size_t rr = t / d.NXC;
-  int k = (int)(rr % d.NZ2), j = (int)(rr / d.NZ2);
+  int m, k, j;
+  size_t t;
+  if (!kept_mode(d, m, k, j, t)) return;
   if (!(in(j, r.js, r.je + 1) && in(k, r.zs, r.ze + 1))) {
-    F2[t] = make_double2(0.0, 0.0);
-    F3[t] = make_double2(0.0, 0.0);
+    // the whole pencil: the scalar's fluxes read the faces of these points, in
+    // physical space, where its range is wider than the velocities'
+    for (int c = m; c < d.NXC; c += d.NKX + 1) {
+      F2[t - m + c] = make_double2(0.0, 0.0);
+      F3[t - m + c] = make_double2(0.0, 0.0);
+    }
     return;
   }
   size_t dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
@@ -950,17 +948,14 @@ __global__ void k_project(Dims d, Metrics M, Ranges r, const double* __restrict_
                           const double2* __restrict__ F3, double2* __restrict__ CU1,
                           double2* __restrict__ CU2, double2* __restrict__ CU3,
                           double2* __restrict__ DIV) {
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  int m = (int)(t % d.NXC);
-  size_t rr = t / d.NXC;
-  int k = (int)(rr % d.NZ2), j = (int)(rr / d.NZ2);
+  int m, k, j;
+  size_t q;
+  if (!kept_mode(d, m, k, j, q)) return;
   if (!(in(j, r.js, r.je) && in(k, r.zs, r.ze))) {
-    DIV[t] = make_double2(0.0, 0.0);
+    DIV[q] = make_double2(0.0, 0.0);
     return;
   }
-  size_t q = t, dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
+  size_t dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
   double w = kx[m];
   double2 p0 = P[q], pjp = P[q + dj], pjm = P[q - dj], pkp = P[q + dk], pkm = P[q - dk];
   double2 u1 = CU1[q], u2 = CU2[q], u3 = CU3[q];
@@ -986,14 +981,10 @@ __global__ void k_project(Dims d, Metrics M, Ranges r, const double* __restrict_
 // CPX += phi / TEMP4 over J = js-1..je+1, K = zs-1..ze+1 (:2460-2466)
 __global__ void k_pupdate(Dims d, Ranges r, const double2* __restrict__ P, double2* __restrict__ CP,
                           const StepState* __restrict__ ss) {
-  int nk = r.ze - r.zs + 3, nj = r.je - r.js + 3;
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t n = (size_t)d.NXC * nk * nj;
-  if (t >= n) return;
-  int m = (int)(t % d.NXC);
-  size_t rr = t / d.NXC;
-  int k = r.zs - 1 + (int)(rr % nk), j = r.js - 1 + (int)(rr / nk);
-  size_t q = fo(d, m, k, j);
+  int m, k, j;
+  size_t q;
+  if (!kept_mode(d, m, k, j, q)) return;
+  if (!(in(j, r.js - 1, r.je + 1) && in(k, r.zs - 1, r.ze + 1))) return;
   const double temp4 = ss->temp4;
   double2 c = CP[q], p = P[q];
   c.x = c.x + p.x / temp4;
@@ -1515,7 +1506,7 @@ __global__ void __launch_bounds__(1024) k_wall_model(Dims d, Metrics M, WallArgs
 static inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 int launch_rhs_fourier(const Dims& d, const Metrics& M, const RhsArgs& a, hipStream_t st) {
-  size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
+  size_t n = kept_modes(d);
   hipLaunchKernelGGL(k_rhs_fourier, dim3(nblk(n, 256)), dim3(256), 0, st, d, M, a);
   EKM_CHECK(hipGetLastError());
   return EKM_OK;
@@ -1612,7 +1603,7 @@ int launch_cfl(const Dims& d, const Metrics& M, const Ranges& r, const double* U
 }
 int launch_faces(const Dims& d, const Metrics& M, const Ranges& r, const double* CU2, const double* CU3,
                  double* F2, double* F3, hipStream_t st) {
-  size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
+  size_t n = kept_modes(d);
   hipLaunchKernelGGL(k_faces, dim3(nblk(n, 256)), dim3(256), 0, st, d, M, r, (const double2*)CU2,
                      (const double2*)CU3, (double2*)F2, (double2*)F3);
   EKM_CHECK(hipGetLastError());
@@ -1635,7 +1626,7 @@ int launch_mg_scatter(const Dims& d, const double* phi, int nmode, int fp32, dou
 int launch_project(const Dims& d, const Metrics& M, const Ranges& r, const double* kx, const double* PHI,
                    const double* F2, const double* F3, double* CU1, double* CU2, double* CU3, double* DIV,
                    hipStream_t st) {
-  size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
+  size_t n = kept_modes(d);
   hipLaunchKernelGGL(k_project, dim3(nblk(n, 256)), dim3(256), 0, st, d, M, r, kx, (const double2*)PHI,
                      (const double2*)F2, (const double2*)F3, (double2*)CU1, (double2*)CU2, (double2*)CU3,
                      (double2*)DIV);
@@ -1644,7 +1635,7 @@ int launch_project(const Dims& d, const Metrics& M, const Ranges& r, const doubl
 }
 int launch_pupdate(const Dims& d, const Ranges& r, const double* PHI, double* CP, const StepState* ss,
                    hipStream_t st) {
-  size_t n = (size_t)d.NXC * (r.ze - r.zs + 3) * (r.je - r.js + 3);
+  size_t n = kept_modes(d);
   hipLaunchKernelGGL(k_pupdate, dim3(nblk(n, 256)), dim3(256), 0, st, d, r, (const double2*)PHI, (double2*)CP,
                      ss);
   EKM_CHECK(hipGetLastError());

@@ -62,12 +62,9 @@ __device__ inline double2 ikx(double kx, double2 f) { return make_double2(-kx * 
 __global__ void k_les_strain(Dims d, Metrics M, Ranges r, const double* __restrict__ kxv, const double2* CU1,
                              const double2* CU2, const double2* CU3, double2* S0, double2* S1, double2* S2,
                              double2* S3, double2* S4, double2* S5) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  const int m = (int)(t % d.NXC);
-  const size_t rr = t / d.NXC;
-  const int k = (int)(rr % d.NZ2), j = (int)(rr / d.NZ2);
+  int m, k, j;
+  size_t t;
+  if (!kept_mode(d, m, k, j, t)) return;
   const size_t dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
   double2 s[6];
   for (int c = 0; c < 6; ++c) s[c] = make_double2(0.0, 0.0);
@@ -242,12 +239,9 @@ __global__ void k_les_ghosts(Dims d, LesFields L, int pass) {
 __global__ void k_les_cf(Dims d, Metrics M, Ranges r, const double* __restrict__ kxv, const double2* C1,
                          const double2* C4, const double2* C5, const double2* C6, double2* CF1, double2* CF2,
                          double2* CF3) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  const int m = (int)(t % d.NXC);
-  const size_t rr = t / d.NXC;
-  const int k = (int)(rr % d.NZ2), j = (int)(rr / d.NZ2);
+  int m, k, j;
+  size_t t;
+  if (!kept_mode(d, m, k, j, t)) return;
   if (!(in(j, r.js, r.je) && in(k, r.zs, r.ze))) return;
   const size_t dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
   const double Jc = JAC(k, j), kx = kxv[m];
@@ -273,12 +267,9 @@ __global__ void k_les_cf(Dims d, Metrics M, Ranges r, const double* __restrict__
 // only on the substeps that recompute it.
 __global__ void k_les_thgrad(Dims d, Metrics M, Ranges r, const double* __restrict__ kxv, const double2* CTH,
                              double2* G0, double2* G1, double2* G2, int full) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  const int m = (int)(t % d.NXC);
-  const size_t rr = t / d.NXC;
-  const int k = (int)(rr % d.NZ2), j = (int)(rr / d.NZ2);
+  int m, k, j;
+  size_t t;
+  if (!kept_mode(d, m, k, j, t)) return;
   const size_t dk = d.NXC, dj = (size_t)d.NXC * d.NZ2;
   double2 g0 = make_double2(0.0, 0.0), g1 = g0, g2 = g0;
   if (in(j, r.js, r.je) && in(k, r.zs, r.ze)) {
@@ -324,12 +315,9 @@ __global__ void k_les_kappa(Dims d, Ranges rt, const double* __restrict__ delta,
 // CFTH -= J i kx (flux)^ on the scalar's interior (:411-419)
 __global__ void k_les_thcf(Dims d, Metrics M, Ranges rt, const double* __restrict__ kxv, const double2* F,
                            double2* CFTH) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t n = (size_t)d.NXC * d.NZ2 * d.NY2;
-  if (t >= n) return;
-  const int m = (int)(t % d.NXC);
-  const size_t rr = t / d.NXC;
-  const int k = (int)(rr % d.NZ2), j = (int)(rr / d.NZ2);
+  int m, k, j;
+  size_t t;
+  if (!kept_mode(d, m, k, j, t)) return;
   if (!(in(j, rt.js, rt.je) && in(k, rt.zs, rt.ze))) return;
   const double a = JAC(k, j) * kxv[m];
   const double2 f = F[t];
@@ -346,7 +334,7 @@ inline unsigned nblk(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
 int les_chan_th_run(const FftPlan& fft, const Dims& d, const Metrics& M, const Ranges& rv, const Ranges& rt,
                     const double* kx, const double* thbar, double* const U[3], double* TH, double* CFTH,
                     const LesFields& L, const LesScratch& w, bool refresh, hipStream_t st) {
-  const size_t nf = (size_t)d.NXC * d.NZ2 * d.NY2, np = d.npts;
+  const size_t nf = kept_modes(d), np = d.npts;
   const long npen = (long)d.plane;
   double* G[3] = {L.S[0], L.S[1], L.S[2]};
   hipLaunchKernelGGL(k_les_thgrad, dim3(nblk(nf, 256)), dim3(256), 0, st, d, M, rv, kx, (const double2*)TH,
@@ -402,7 +390,7 @@ int les_chan_th_run(const FftPlan& fft, const Dims& d, const Metrics& M, const R
 int les_chan_run(const FftPlan& fft, const Dims& d, const Metrics& M, const Ranges& r, const double* kx,
                  double* const U[3], double* const CF[3], const LesFields& L, const LesScratch& w, bool refresh,
                  hipStream_t st) {
-  const size_t nf = (size_t)d.NXC * d.NZ2 * d.NY2, np = d.npts;
+  const size_t nf = kept_modes(d), np = d.npts;
   const long npen = (long)d.plane;
   hipLaunchKernelGGL(k_les_strain, dim3(nblk(nf, 256)), dim3(256), 0, st, d, M, r, kx, (const double2*)U[0],
                      (const double2*)U[1], (const double2*)U[2], (double2*)L.S[0], (double2*)L.S[1],
