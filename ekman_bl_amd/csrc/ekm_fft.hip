@@ -29,6 +29,12 @@ namespace {
 constexpr int kWaves = 4;  // wavefronts per block
 constexpr int kBlock = 64 * kWaves;
 
+// the fields of one launch of transforms (blockIdx.y picks one)
+constexpr int kFftFields = 6;
+struct FftFields {
+  double* v[kFftFields];
+};
+
 __device__ inline double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
@@ -152,10 +158,11 @@ __device__ inline void dif_any(double2 (&z)[R], int GW, int M, int lanep, const 
 __device__ inline int bitrev(int e, int logm) { return (int)(__brev((unsigned)e) >> (32 - logm)); }
 
 template <int R>
-__global__ void __launch_bounds__(kBlock) k_fft_fwd(double* __restrict__ v, long npencil, int nx, int logm,
+__global__ void __launch_bounds__(kBlock) k_fft_fwd(FftFields fl, long npencil, int nx, int logm,
                                                     const double2* __restrict__ tw,
                                                     const double2* __restrict__ tw2) {
   extern __shared__ double2 lds[];
+  double* __restrict__ v = fl.v[blockIdx.y];
   const int M = nx >> 1, GW = M < 64 ? M : 64, PW = 64 / GW;  // pencils per wave
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lanep = lane % GW, sub = lane / GW;
@@ -201,10 +208,11 @@ __global__ void __launch_bounds__(kBlock) k_fft_fwd(double* __restrict__ v, long
 }
 
 template <int R>
-__global__ void __launch_bounds__(kBlock) k_fft_inv(double* __restrict__ v, long npencil, int nx, int logm,
+__global__ void __launch_bounds__(kBlock) k_fft_inv(FftFields fl, long npencil, int nx, int logm,
                                                     const double2* __restrict__ tw,
                                                     const double2* __restrict__ tw2) {
   extern __shared__ double2 lds[];
+  double* __restrict__ v = fl.v[blockIdx.y];
   const int M = nx >> 1, GW = M < 64 ? M : 64, PW = 64 / GW;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lanep = lane % GW, sub = lane / GW;
@@ -267,22 +275,31 @@ __global__ void __launch_bounds__(kBlock) k_fft_inv(double* __restrict__ v, long
 // transform is linear, so the two differ by rounding only.
 #define MET(arr, k, j, f) M.arr[mf(d, k, j, f)]
 template <int R, bool LES>
-__global__ void __launch_bounds__(kBlock) k_flux_accum(Dims d, Metrics M, Ranges rg, const double* __restrict__ U1,
-                                                       const double* __restrict__ Q, const double* __restrict__ U2b,
-                                                       const double* __restrict__ U3b, double nu,
-                                                       const double* __restrict__ kxv, double2* __restrict__ CF,
-                                                       double2* __restrict__ CR, const double* __restrict__ temp5p, int logm,
-                                                       const double2* __restrict__ tw,
-                                                       const double2* __restrict__ tw2,
-                                                       const double* __restrict__ nut,
-                                                       const double* __restrict__ gl) {
+__global__ void __launch_bounds__(kBlock) k_flux_accum(Dims d, Metrics M, FluxBatch fb, const double* __restrict__ U1,
+                                                       const double* __restrict__ U2b, const double* __restrict__ U3b,
+                                                       const double* __restrict__ kxv, const double* __restrict__ temp5p,
+                                                       int logm, const double2* __restrict__ tw,
+                                                       const double2* __restrict__ tw2) {
   extern __shared__ double2 lds[];
+  // the same pencils of all fields run side by side on one XCD (workgroups are
+  // dealt to the 8 XCDs round robin): the advecting velocities U1, U2b, U3b and
+  // the eddy viscosity, which every field reads, come from its L2 after the first
+  const int slot = blockIdx.x >> 3, fi = slot % fb.n;
+  const long pblk = (long)(slot / fb.n) * 8 + (blockIdx.x & 7);
+  const FluxField& ff = fb.f[fi];
+  const Ranges rg = ff.rg;
+  const double nu = ff.nu;
+  const double* __restrict__ Q = ff.Q;
+  const double* __restrict__ nut = ff.nut;
+  const double* __restrict__ gl = ff.gl;
+  double2* __restrict__ CF = ff.CF;
+  double2* __restrict__ CR = ff.CR;
   const int nx = d.NX, M2 = nx >> 1, GW = M2 < 64 ? M2 : 64, PW = 64 / GW;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lanep = lane % GW, sub = lane / GW;
   const int nk = rg.ze - rg.zs + 1, nj = rg.je - rg.js + 1;
   const long npen = (long)nk * nj;
-  const long pen = ((long)blockIdx.x * kWaves + wave) * PW + sub;
+  const long pen = (pblk * kWaves + wave) * PW + sub;
   const bool live = pen < npen;
   const int k = rg.zs + (int)(live ? pen % nk : 0), j = rg.js + (int)(live ? pen / nk : 0);
   const size_t dj = (size_t)d.NX2 * d.NZ2, dk = d.NX2;
@@ -415,31 +432,30 @@ __global__ void __launch_bounds__(kBlock) k_flux_accum(Dims d, Metrics M, Ranges
 #undef MET
 
 template <int R>
-int launch_flux_accum_r(const FftPlan& p, const Dims& d, const Metrics& M, const Ranges& rg, const double* U1,
-                        const double* Q, const double* U2b, const double* U3b, double nu, const double* kx,
-                        double* CF, double* CR, const double* temp5, const double* nut, const double* gl, hipStream_t st) {
+int launch_flux_accum_r(const FftPlan& p, const Dims& d, const Metrics& M, const FluxBatch& fb, const double* U1,
+                        const double* U2b, const double* U3b, const double* kx, const double* temp5, hipStream_t st) {
   const int M2 = p.nx / 2, GW = M2 < 64 ? M2 : 64, PW = 64 / GW;
-  const long npen = (long)(rg.ze - rg.zs + 1) * (rg.je - rg.js + 1);
+  long npen = 0;
+  for (int f = 0; f < fb.n; ++f)
+    npen = std::max(npen, (long)(fb.f[f].rg.ze - fb.f[f].rg.zs + 1) * (fb.f[f].rg.je - fb.f[f].rg.js + 1));
   if (npen <= 0) return EKM_OK;
   const long per_block = (long)kWaves * PW;
-  const long nb = (npen + per_block - 1) / per_block;
+  const long nb = ((npen + per_block - 1) / per_block + 7) / 8 * 8 * fb.n;
   const size_t lds = (size_t)2 * kWaves * PW * M2 * sizeof(double2);
   int logm = 0;
   while ((1 << logm) < M2) ++logm;
-  if (nut)
-    hipLaunchKernelGGL((k_flux_accum<R, true>), dim3((unsigned)nb), dim3(kBlock), lds, st, d, M, rg, U1, Q, U2b, U3b,
-                       nu, kx, (double2*)CF, (double2*)CR, temp5, logm, (const double2*)p.tw, (const double2*)p.tw2,
-                       nut, gl);
+  if (fb.f[0].nut)
+    hipLaunchKernelGGL((k_flux_accum<R, true>), dim3((unsigned)nb), dim3(kBlock), lds, st, d, M, fb, U1, U2b, U3b, kx,
+                       temp5, logm, (const double2*)p.tw, (const double2*)p.tw2);
   else
-    hipLaunchKernelGGL((k_flux_accum<R, false>), dim3((unsigned)nb), dim3(kBlock), lds, st, d, M, rg, U1, Q, U2b,
-                       U3b, nu, kx, (double2*)CF, (double2*)CR, temp5, logm, (const double2*)p.tw,
-                       (const double2*)p.tw2, nullptr, nullptr);
+    hipLaunchKernelGGL((k_flux_accum<R, false>), dim3((unsigned)nb), dim3(kBlock), lds, st, d, M, fb, U1, U2b, U3b, kx,
+                       temp5, logm, (const double2*)p.tw, (const double2*)p.tw2);
   EKM_CHECK(hipGetLastError());
   return EKM_OK;
 }
 
 template <int R>
-int launch_pair(bool fwd, const FftPlan& p, double* v, long npencil, hipStream_t st) {
+int launch_pair(bool fwd, const FftPlan& p, const FftFields& v, int nf, long npencil, hipStream_t st) {
   const int M = p.nx / 2, GW = M < 64 ? M : 64, PW = 64 / GW;
   const long per_block = (long)kWaves * PW;
   const long nb = (npencil + per_block - 1) / per_block;
@@ -447,22 +463,25 @@ int launch_pair(bool fwd, const FftPlan& p, double* v, long npencil, hipStream_t
   int logm = 0;
   while ((1 << logm) < M) ++logm;
   if (fwd)
-    hipLaunchKernelGGL(k_fft_fwd<R>, dim3((unsigned)nb), dim3(kBlock), lds, st, v, npencil, p.nx, logm,
+    hipLaunchKernelGGL(k_fft_fwd<R>, dim3((unsigned)nb, (unsigned)nf), dim3(kBlock), lds, st, v, npencil, p.nx, logm,
                        (const double2*)p.tw, (const double2*)p.tw2);
   else
-    hipLaunchKernelGGL(k_fft_inv<R>, dim3((unsigned)nb), dim3(kBlock), lds, st, v, npencil, p.nx, logm,
+    hipLaunchKernelGGL(k_fft_inv<R>, dim3((unsigned)nb, (unsigned)nf), dim3(kBlock), lds, st, v, npencil, p.nx, logm,
                        (const double2*)p.tw, (const double2*)p.tw2);
   EKM_CHECK(hipGetLastError());
   return EKM_OK;
 }
 
-int launch(bool fwd, const FftPlan& p, double* v, long npencil, hipStream_t st) {
-  if (npencil <= 0) return EKM_OK;
+int launch(bool fwd, const FftPlan& p, double* const* f, int nf, long npencil, hipStream_t st) {
+  if (npencil <= 0 || nf <= 0) return EKM_OK;
+  if (nf > kFftFields) return EKM_ERR_ARG;
+  FftFields v{};
+  for (int c = 0; c < nf; ++c) v.v[c] = f[c];
   const int M = p.nx / 2;
-  if (M <= 64) return launch_pair<1>(fwd, p, v, npencil, st);
-  if (M == 128) return launch_pair<2>(fwd, p, v, npencil, st);
-  if (M == 256) return launch_pair<4>(fwd, p, v, npencil, st);
-  return launch_pair<8>(fwd, p, v, npencil, st);
+  if (M <= 64) return launch_pair<1>(fwd, p, v, nf, npencil, st);
+  if (M == 128) return launch_pair<2>(fwd, p, v, nf, npencil, st);
+  if (M == 256) return launch_pair<4>(fwd, p, v, nf, npencil, st);
+  return launch_pair<8>(fwd, p, v, nf, npencil, st);
 }
 
 }  // namespace
@@ -503,19 +522,27 @@ void fft_plan_free(FftPlan& p) {
   p.tw = p.tw2 = nullptr;
 }
 
-int fft_forward(const FftPlan& p, double* v, long npencil, hipStream_t st) { return launch(true, p, v, npencil, st); }
+int fft_forward(const FftPlan& p, double* v, long npencil, hipStream_t st) { return launch(true, p, &v, 1, npencil, st); }
 
-int fft_inverse(const FftPlan& p, double* v, long npencil, hipStream_t st) { return launch(false, p, v, npencil, st); }
+int fft_inverse(const FftPlan& p, double* v, long npencil, hipStream_t st) { return launch(false, p, &v, 1, npencil, st); }
 
-int launch_flux_accum(const FftPlan& p, const Dims& d, const Metrics& M, const Ranges& r, const double* U1,
-                      const double* Q, const double* U2b, const double* U3b, double nu, const double* kx, double* CF,
-                      double* CR, const double* temp5, hipStream_t st, const double* nut, const double* gl) {
+int fft_forward_n(const FftPlan& p, double* const* v, int n, long npencil, hipStream_t st) {
+  return launch(true, p, v, n, npencil, st);
+}
+
+int fft_inverse_n(const FftPlan& p, double* const* v, int n, long npencil, hipStream_t st) {
+  return launch(false, p, v, n, npencil, st);
+}
+
+int launch_flux_accum(const FftPlan& p, const Dims& d, const Metrics& M, const FluxBatch& fb, const double* U1,
+                      const double* U2b, const double* U3b, const double* kx, const double* temp5, hipStream_t st) {
   const int M2 = p.nx / 2;
-  if (nut && !gl) return EKM_ERR_ARG;
-  if (M2 <= 64) return launch_flux_accum_r<1>(p, d, M, r, U1, Q, U2b, U3b, nu, kx, CF, CR, temp5, nut, gl, st);
-  if (M2 == 128) return launch_flux_accum_r<2>(p, d, M, r, U1, Q, U2b, U3b, nu, kx, CF, CR, temp5, nut, gl, st);
-  if (M2 == 256) return launch_flux_accum_r<4>(p, d, M, r, U1, Q, U2b, U3b, nu, kx, CF, CR, temp5, nut, gl, st);
-  return launch_flux_accum_r<8>(p, d, M, r, U1, Q, U2b, U3b, nu, kx, CF, CR, temp5, nut, gl, st);
+  for (int f = 0; f < fb.n; ++f)
+    if (!fb.f[f].nut != !fb.f[0].nut || (fb.f[f].nut && !fb.f[f].gl)) return EKM_ERR_ARG;
+  if (M2 <= 64) return launch_flux_accum_r<1>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
+  if (M2 == 128) return launch_flux_accum_r<2>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
+  if (M2 == 256) return launch_flux_accum_r<4>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
+  return launch_flux_accum_r<8>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -137,13 +137,27 @@ void fft_plan_free(FftPlan& p);
 // in-place transforms of npencil pencils of stride NX+2
 int fft_forward(const FftPlan& p, double* v, long npencil, hipStream_t st);
 int fft_inverse(const FftPlan& p, double* v, long npencil, hipStream_t st);
-// fused flux -> forward transform -> CF/CR accumulation of one transported
-// field; nut (with its cross-term metric gl) adds the subgrid viscosity's
-// cross terms
-int launch_flux_accum(const FftPlan& p, const Dims& d, const Metrics& M, const Ranges& r, const double* U1,
-                      const double* Q, const double* U2b, const double* U3b, double nu, const double* kx, double* CF,
-                      double* CR, const double* temp5, hipStream_t st, const double* nut = nullptr,
-                      const double* gl = nullptr);
+// the same of n fields (at most 6) in one launch
+int fft_forward_n(const FftPlan& p, double* const* v, int n, long npencil, hipStream_t st);
+int fft_inverse_n(const FftPlan& p, double* const* v, int n, long npencil, hipStream_t st);
+// fused flux -> forward transform -> CF/CR accumulation of the transported
+// fields, in one launch; nut (all fields or none) with its cross-term metric
+// gl adds the subgrid viscosity's cross terms
+struct FluxField {
+  const double* Q;
+  double2* CF;
+  double2* CR;
+  const double* nut;
+  const double* gl;
+  double nu;
+  Ranges rg;
+};
+struct FluxBatch {
+  int n;
+  FluxField f[4];
+};
+int launch_flux_accum(const FftPlan& p, const Dims& d, const Metrics& M, const FluxBatch& fb, const double* U1,
+                      const double* U2b, const double* U3b, const double* kx, const double* temp5, hipStream_t st);
 
 // ---- multigrid --------------------------------------------------------------
 struct HostMetrics;

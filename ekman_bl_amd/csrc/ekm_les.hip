@@ -340,8 +340,8 @@ int les_chan_th_run(const FftPlan& fft, const Dims& d, const Metrics& M, const R
   hipLaunchKernelGGL(k_les_thgrad, dim3(nblk(nf, 256)), dim3(256), 0, st, d, M, rv, kx, (const double2*)TH,
                      (double2*)G[0], (double2*)G[1], (double2*)G[2], refresh ? 1 : 0);
   EKM_CHECK(hipGetLastError());
-  for (int c = 0; c < (refresh ? 3 : 1); ++c) {
-    const int e = fft_inverse(fft, G[c], npen, st);
+  {
+    const int e = fft_inverse_n(fft, G, refresh ? 3 : 1, npen, st);
     if (e != EKM_OK) return e;
   }
   if (refresh) {
@@ -396,14 +396,14 @@ int les_chan_run(const FftPlan& fft, const Dims& d, const Metrics& M, const Rang
                      (const double2*)U[1], (const double2*)U[2], (double2*)L.S[0], (double2*)L.S[1],
                      (double2*)L.S[2], (double2*)L.S[3], (double2*)L.S[4], (double2*)L.S[5]);
   EKM_CHECK(hipGetLastError());
-  for (int c = 0; c < 6; ++c) {
-    const int e = fft_inverse(fft, L.S[c], npen, st);
+  {
+    const int e = fft_inverse_n(fft, L.S, 6, npen, st);
     if (e != EKM_OK) return e;
   }
   hipLaunchKernelGGL(k_les_sabs, dim3(nblk(np, 256)), dim3(256), 0, st, d, r, L);
   EKM_CHECK(hipGetLastError());
-  for (int c = 0; c < 3; ++c) {
-    const int e = fft_inverse(fft, U[c], npen, st);
+  {
+    const int e = fft_inverse_n(fft, U, 3, npen, st);
     if (e != EKM_OK) return e;
   }
   if (refresh) {
@@ -437,8 +437,9 @@ int les_chan_run(const FftPlan& fft, const Dims& d, const Metrics& M, const Rang
     hipLaunchKernelGGL(k_les_ghosts, dim3(nblk(ng, 256)), dim3(256), 0, st, d, L, pass);
     EKM_CHECK(hipGetLastError());
   }
-  for (int c : {0, 3, 4, 5}) {
-    const int e = fft_forward(fft, L.S[c], npen, st);
+  {
+    double* v[4] = {L.S[0], L.S[3], L.S[4], L.S[5]};
+    const int e = fft_forward_n(fft, v, 4, npen, st);
     if (e != EKM_OK) return e;
   }
   hipLaunchKernelGGL(k_les_cf, dim3(nblk(nf, 256)), dim3(256), 0, st, d, M, r, kx, (const double2*)L.S[0],

@@ -956,30 +956,36 @@ static int enqueue_substep(ekm_solver* s, const SubstepPlan& q, bool timed) {
   if (q.les_on) {
     TRY(les_chan_run(s->fft, d, s->M, s->rv, s->kx, s->U, s->CF, s->les, s->lesw, q.refresh, st));
   } else {
-    for (int f = 0; f < 3; ++f) TRY(inv(s, s->U[f]));
+    double* v[4] = {s->U[0], s->U[1], s->U[2], s->TH};
+    TRY(fft_inverse_n(s->fft, v, th ? 4 : 3, (long)d.plane, st));
   }
   // the scalar's subgrid model (:650-654), which leaves the scalar in
   // physical space, or the scalar to physical space
   if (th && q.les_on) {
     TRY(les_chan_th_run(s->fft, d, s->M, s->rv, s->rt, s->kx, s->thbar, s->U, s->TH, s->CFTH, s->les, s->lesw,
                         q.refresh_th, st));
-  } else if (th) {
-    TRY(inv(s, s->TH));
   }
   // momentum fluxes (:683-1161)
   TRY(launch_contravariant(d, s->M, s->rv, s->U[1], s->U[2], s->U2b, s->U3b, st));
   // (with the model: its eddy-viscosity cross terms, :990-1120)
   const double* temp5 = SS_PTR(s, temp5);
-  for (int f = 0; f < 3; ++f) {
-    TRY(launch_flux_accum(s->fft, d, s->M, s->rv, s->U[0], s->U[f], s->U2b, s->U3b, p.nu, s->kx, s->CF[f],
-                          s->R[f], temp5, st, q.les_on ? s->les.nut : nullptr,
-                          q.les_on ? les_metric(s, f, 2) : nullptr));
+  // (the scalar's: :1169-1625)
+  FluxBatch fb;
+  fb.n = th ? 4 : 3;
+  for (int f = 0; f < fb.n; ++f) {
+    const bool v = f < 3;
+    fb.f[f].Q = v ? s->U[f] : s->TH;
+    fb.f[f].CF = (double2*)(v ? s->CF[f] : s->CFTH);
+    fb.f[f].CR = (double2*)(v ? s->R[f] : s->RTH);
+    fb.f[f].nut = !q.les_on ? nullptr : v ? s->les.nut : s->les.kappa;
+    fb.f[f].gl = !q.les_on ? nullptr : v ? les_metric(s, f, 2) : s->M.g12;
+    fb.f[f].nu = v ? p.nu : p.nu / p.pr;
+    fb.f[f].rg = v ? s->rv : s->rt;
   }
-  for (int f = 0; f < 3; ++f) TRY(inv(s, s->R[f]));
-  if (th) {  // (:1169-1625)
-    TRY(launch_flux_accum(s->fft, d, s->M, s->rt, s->U[0], s->TH, s->U2b, s->U3b, p.nu / p.pr, s->kx, s->CFTH,
-                          s->RTH, temp5, st, q.les_on ? s->les.kappa : nullptr, q.les_on ? s->M.g12 : nullptr));
-    TRY(inv(s, s->RTH));
+  TRY(launch_flux_accum(s->fft, d, s->M, fb, s->U[0], s->U2b, s->U3b, s->kx, temp5, st));
+  {
+    double* r[4] = {s->R[0], s->R[1], s->R[2], s->RTH};
+    TRY(fft_inverse_n(s->fft, r, fb.n, (long)d.plane, st));
   }
   // LES_WALL_MODEL (:1687-1691) from the velocities entering the implicit
   // solves, in physical space here as there
@@ -1012,8 +1018,10 @@ static int enqueue_substep(ekm_solver* s, const SubstepPlan& q, bool timed) {
     TRY(launch_dt_update(s->ss, st));
   }
   // back to Fourier space and project (:2421-2455)
-  for (int f = 0; f < 3; ++f) TRY(fwd(s, s->U[f]));
-  if (th) TRY(fwd(s, s->TH));
+  {
+    double* v[4] = {s->U[0], s->U[1], s->U[2], s->TH};
+    TRY(fft_forward_n(s->fft, v, th ? 4 : 3, (long)d.plane, st));
+  }
   TRY(rem_div(s, q.guess_on ? SS_PTR(s, guess) : nullptr, timed, q.guess_on == 2));
   // pressure update (:2460-2466)
   TRY(launch_pupdate(d, s->rv, s->PHI, s->P, s->ss, st));
