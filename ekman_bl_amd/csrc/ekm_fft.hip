@@ -17,6 +17,7 @@
 // The inverse builds Z_k from the modes in registers and runs the same
 // stages on the conjugate.  Loads and stores are contiguous across lanes.
 #include "ekm_internal.h"
+#include "ekm_kernels.h"
 
 #include <cmath>
 #include <cstdio>
@@ -207,23 +208,16 @@ __global__ void __launch_bounds__(kBlock) k_fft_fwd(FftFields fl, long npencil, 
   }
 }
 
+// The inverse transform of one pencil up to its last stage: on return z[r] of
+// lane lanep is the conjugate of the value pair (u_2k, u_2k+1) with k =
+// bitrev(lanep + GW r).
+// Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/NX} (X_k - conj X_{M-k}), k < M,
+// conjugated: the inverse transform is conj(DFT(conj Z))
 template <int R>
-__global__ void __launch_bounds__(kBlock) k_fft_inv(FftFields fl, long npencil, int nx, int logm,
-                                                    const double2* __restrict__ tw,
-                                                    const double2* __restrict__ tw2) {
-  extern __shared__ double2 lds[];
-  double* __restrict__ v = fl.v[blockIdx.y];
-  const int M = nx >> 1, GW = M < 64 ? M : 64, PW = 64 / GW;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lanep = lane % GW, sub = lane / GW;
-  const long pen = ((long)blockIdx.x * kWaves + wave) * PW + sub;
-  const bool live = pen < npencil;
-  const int stride = nx + 2, nkx = nx / 3;
-  const double2* X = reinterpret_cast<const double2*>(v + (live ? pen : 0) * stride);
-  // Z_k = (X_k + conj X_{M-k}) + i e^{+2 pi i k/NX} (X_k - conj X_{M-k}), k < M,
-  // conjugated: the inverse transform is conj(DFT(conj Z))
+__device__ inline void inverse_stages(double2 (&z)[R], const double2* __restrict__ X, bool live, int nx, int lanep,
+                                      const double2* __restrict__ tw, const double2* __restrict__ tw2) {
+  const int M = nx >> 1, GW = M < 64 ? M : 64, nkx = nx / 3;
   const LaneTw lt = lane_twiddles(lanep, M, tw);
-  double2 z[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int k = lanep + GW * r, b = M - k;
@@ -240,19 +234,105 @@ __global__ void __launch_bounds__(kBlock) k_fft_inv(FftFields fl, long npencil, 
     z[r] = make_double2(e.x - o.y, -(e.y + o.x));
   }
   dif_any<R>(z, GW, M, lanep, tw, lt);
-  double2* Z = lds + (size_t)(wave * PW + sub) * M;
+}
+
+// z into natural order in the pencil's LDS slice, for this wavefront to read
+template <int R>
+__device__ inline void to_natural(const double2 (&z)[R], double2* Z, int GW, int lanep, int logm) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    double2 t = z[r];
-    t.y = -t.y;
-    Z[bitrev(lanep + GW * r, logm)] = t;
-  }
+  for (int r = 0; r < R; ++r) Z[bitrev(lanep + GW * r, logm)] = make_double2(z[r].x, -z[r].y);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+template <int R>
+__global__ void __launch_bounds__(kBlock) k_fft_inv(FftFields fl, long npencil, int nx, int logm,
+                                                    const double2* __restrict__ tw,
+                                                    const double2* __restrict__ tw2) {
+  extern __shared__ double2 lds[];
+  double* __restrict__ v = fl.v[blockIdx.y];
+  const int M = nx >> 1, GW = M < 64 ? M : 64, PW = 64 / GW;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lanep = lane % GW, sub = lane / GW;
+  const long pen = ((long)blockIdx.x * kWaves + wave) * PW + sub;
+  const bool live = pen < npencil;
+  double2 z[R];
+  inverse_stages<R>(z, reinterpret_cast<const double2*>(v + (live ? pen : 0) * (nx + 2)), live, nx, lanep, tw, tw2);
+  double2* Z = lds + (size_t)(wave * PW + sub) * M;
+  to_natural<R>(z, Z, GW, lanep, logm);
   if (!live) return;
-  double2* dst = reinterpret_cast<double2*>(v + pen * stride);
+  double2* dst = reinterpret_cast<double2*>(v + pen * (nx + 2));
   for (int k = lanep; k <= M; k += GW) dst[k] = (k < M) ? Z[k] : make_double2(0.0, 0.0);
+}
+
+// The right-hand sides R of the implicit fields to physical space, and with
+// them the explicit half of their Crank-Nicolson operators (src/duct.F90:
+// 1334-1400 and the velocities' analogues): S = R - J U and
+// R' = S/2 + J U + TEMP1 dz(G11 dz U) [+ H_BAR/2 dz(nu_T gz dz U)], so that R
+// does not go through memory between the two.  Pencils outside a field's
+// range are transformed only.  Bound by memory: 2/3 of a pass (the kept modes)
+// and U read, S and R' written per field.
+template <int R, bool LES>
+__global__ void __launch_bounds__(kBlock) k_inv_pre(Dims d, Metrics M, const AdiField* __restrict__ fs, AdiT1 t1s,
+                                                    int logm, const double2* __restrict__ tw,
+                                                    const double2* __restrict__ tw2) {
+  extern __shared__ double2 lds[];
+  const AdiField& F = fs[blockIdx.y];
+  const Ranges r = F.r;
+  const int nx = d.NX, M2 = nx >> 1, GW = M2 < 64 ? M2 : 64, PW = 64 / GW;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lanep = lane % GW, sub = lane / GW;
+  const long pen = ((long)blockIdx.x * kWaves + wave) * PW + sub;
+  const bool live = pen < (long)d.plane;
+  const size_t row = (size_t)d.NX2 * (size_t)(live ? pen : 0);
+  double2 z[R];
+  inverse_stages<R>(z, reinterpret_cast<const double2*>(F.R + row), live, nx, lanep, tw, tw2);
+  double2* Z = lds + (size_t)(wave * PW + sub) * M2;
+  to_natural<R>(z, Z, GW, lanep, logm);
+  if (!live) return;
+  double2* __restrict__ dst = reinterpret_cast<double2*>(F.R + row);
+  const int k = (int)(pen % d.NZ2), j = (int)(pen / d.NZ2);
+  if (k < r.zs || k > r.ze || j < r.js || j > r.je) {
+    for (int c = lanep; c <= M2; c += GW) dst[c] = (c < M2) ? Z[c] : make_double2(0.0, 0.0);
+    return;
+  }
+  const double t1 = t1s.ss->temp1 / t1s.div[blockIdx.y];
+  const double Jc = M.jac[mi(d, k, j)], gp = M.g11[mf(d, k + 1, j, 2)], gm = M.g11[mf(d, k, j, 2)];
+  double t2 = 0.0, lp = 0.0, lm = 0.0;
+  if constexpr (LES) {
+    t2 = t1s.ss->hb / 2.0;
+    lp = F.gz[mf(d, k + 1, j, 2)];
+    lm = F.gz[mf(d, k, j, 2)];
+  }
+  const int dk = d.NX2 / 2;  // a row of k, in pairs
+  const double2* __restrict__ U = reinterpret_cast<const double2*>(F.U + row);
+  double2* __restrict__ S = reinterpret_cast<double2*>(F.S + row);
+  const double2* __restrict__ N = LES ? reinterpret_cast<const double2*>(F.nut + row) : nullptr;
+  auto half = [&](double rr, double u, double up, double um, double nc, double np, double nm, double& s) {
+    s = rr - Jc * u;
+    double v = 0.5 * s + Jc * u + t1 * (gp * (up - u) - gm * (u - um));
+    if constexpr (LES) v = v + t2 * (0.5 * (np + nc) * (lp * (up - u)) - 0.5 * (nc + nm) * (lm * (u - um)));
+    return v;
+  };
+#pragma unroll 2
+  for (int i = 0; i < R; ++i) {
+    const int c = lanep + GW * i;
+    const double2 u = U[c], up = U[c + dk], um = U[c - dk];
+    double2 nc = make_double2(0.0, 0.0), np = nc, nm = nc;
+    if constexpr (LES) {
+      nc = N[c];
+      np = N[c + dk];
+      nm = N[c - dk];
+    }
+    const double2 rr = Z[c];
+    double2 s, v;
+    v.x = half(rr.x, u.x, up.x, um.x, nc.x, np.x, nm.x, s.x);
+    v.y = half(rr.y, u.y, up.y, um.y, nc.y, np.y, nm.y, s.y);
+    S[c] = s;
+    dst[c] = v;
+  }
+  if (lanep == 0) S[M2] = dst[M2] = make_double2(0.0, 0.0);  // the padding
 }
 
 // Fused nonlinear-flux stage of one transported field Q (RK_DUCT
@@ -455,6 +535,24 @@ int launch_flux_accum_r(const FftPlan& p, const Dims& d, const Metrics& M, const
 }
 
 template <int R>
+int launch_inv_pre_r(const FftPlan& p, const Dims& d, const Metrics& M, const AdiField* fs, int nf, const AdiT1& t1,
+                     bool les, hipStream_t st) {
+  const int M2 = p.nx / 2, GW = M2 < 64 ? M2 : 64, PW = 64 / GW;
+  const long per_block = (long)kWaves * PW, nb = ((long)d.plane + per_block - 1) / per_block;
+  const size_t lds = (size_t)kWaves * PW * M2 * sizeof(double2);
+  int logm = 0;
+  while ((1 << logm) < M2) ++logm;
+  if (les)
+    hipLaunchKernelGGL((k_inv_pre<R, true>), dim3((unsigned)nb, (unsigned)nf), dim3(kBlock), lds, st, d, M, fs, t1, logm,
+                       (const double2*)p.tw, (const double2*)p.tw2);
+  else
+    hipLaunchKernelGGL((k_inv_pre<R, false>), dim3((unsigned)nb, (unsigned)nf), dim3(kBlock), lds, st, d, M, fs, t1, logm,
+                       (const double2*)p.tw, (const double2*)p.tw2);
+  EKM_CHECK(hipGetLastError());
+  return EKM_OK;
+}
+
+template <int R>
 int launch_pair(bool fwd, const FftPlan& p, const FftFields& v, int nf, long npencil, hipStream_t st) {
   const int M = p.nx / 2, GW = M < 64 ? M : 64, PW = 64 / GW;
   const long per_block = (long)kWaves * PW;
@@ -543,6 +641,15 @@ int launch_flux_accum(const FftPlan& p, const Dims& d, const Metrics& M, const F
   if (M2 == 128) return launch_flux_accum_r<2>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
   if (M2 == 256) return launch_flux_accum_r<4>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
   return launch_flux_accum_r<8>(p, d, M, fb, U1, U2b, U3b, kx, temp5, st);
+}
+
+int launch_inv_pre(const FftPlan& p, const Dims& d, const Metrics& M, const AdiField* fs, int nf, const AdiT1& t1,
+                   bool les, hipStream_t st) {
+  const int M2 = p.nx / 2;
+  if (M2 <= 64) return launch_inv_pre_r<1>(p, d, M, fs, nf, t1, les, st);
+  if (M2 == 128) return launch_inv_pre_r<2>(p, d, M, fs, nf, t1, les, st);
+  if (M2 == 256) return launch_inv_pre_r<4>(p, d, M, fs, nf, t1, les, st);
+  return launch_inv_pre_r<8>(p, d, M, fs, nf, t1, les, st);
 }
 
 // ---------------------------------------------------------------------------

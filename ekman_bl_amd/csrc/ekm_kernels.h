@@ -50,7 +50,13 @@ struct AdiT1 {
   const StepState* ss;
   double div[kAdiMaxFields];
 };
-// The ADI sweeps of nf independent fields in one set of launches; fs: nf
+// The fields' right-hand sides R to physical space and their explicit half
+// operators (S, and R for the sweeps), in one launch (ekm_fft.hip); les: the
+// fields carry an eddy viscosity
+int launch_inv_pre(const FftPlan& p, const Dims& d, const Metrics& M, const AdiField* fs, int nf, const AdiT1& t1,
+                   bool les, hipStream_t st);
+// The ADI sweeps of nf independent fields in one set of launches (after
+// launch_inv_pre); fs: nf
 // descriptors in device memory, hf the same on the host (for the grid sizes).
 // th_corners applies the scalar corner rows to field th_field afterwards.
 int launch_adi_batch(const Dims& d, const Metrics& M, const AdiField* fs, const AdiField* hf, int nf,

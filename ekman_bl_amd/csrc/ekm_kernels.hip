@@ -159,34 +159,6 @@ __global__ void k_contravariant(Dims d, Metrics M, Ranges r, const double* __res
 // ADI: explicit half before the y sweep (:1334-1371, :1640-1665, ...)
 // S = R - J U;  R = S/2 + J U + t1 [G11(K+1)(U(K+1)-U) - G11(K)(U-U(K-1))]
 // ---------------------------------------------------------------------------
-__global__ void k_adi_pre(Dims d, Metrics M, const AdiField* __restrict__ fs, AdiT1 t1s) {
-  const AdiField& F = fs[blockIdx.y];
-  const Ranges r = F.r;
-  const double t1 = t1s.ss->temp1 / t1s.div[blockIdx.y];
-  const double* __restrict__ U = F.U;
-  double* __restrict__ R = F.R;
-  double* __restrict__ S = F.S;
-  int nk = r.ze - r.zs + 1, nj = r.je - r.js + 1;
-  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t n = (size_t)d.NX2 * nk * nj;
-  if (t >= n) return;
-  int i = (int)(t % d.NX2);
-  size_t rr = t / d.NX2;
-  int k = r.zs + (int)(rr % nk), j = r.js + (int)(rr / nk);
-  size_t q = ph(d, i, k, j), dk = d.NX2;
-  double Jc = JAC(k, j), u = U[q];
-  double s = R[q] - Jc * u;
-  S[q] = s;
-  double rv = 0.5 * s + Jc * u + t1 * (G11(k + 1, j, 2) * (U[q + dk] - u) - G11(k, j, 2) * (u - U[q - dk]));
-  if (F.nut) {  // subgrid viscosity, z direction (:1667-1680 and analogues)
-    const double* __restrict__ nut = F.nut;
-    const double* __restrict__ gz = F.gz;
-    const double t2 = t1s.ss->hb / 2.0, nc = nut[q];
-    rv = rv + t2 * (0.5 * (nut[q + dk] + nc) * (gz[mf(d, k + 1, j, 2)] * (U[q + dk] - u)) -
-                    0.5 * (nc + nut[q - dk]) * (gz[mf(d, k, j, 2)] * (u - U[q - dk])));
-  }
-  R[q] = rv;
-}
 
 // Per-line factorisation of one sweep (THOMAS_REAL forward elimination,
 // src/boundary.F90:53-84, with the rows of the APPLY_BC_* routines).  dir 0:
@@ -1523,7 +1495,7 @@ int launch_adi_batch(const Dims& d, const Metrics& M, const AdiField* fs, const 
   if (nf < 1 || nf > kAdiMaxFields) return EKM_ERR_ARG;
   const int bs = tn.adi_block;
   if (d.NY + 2 > kLuMaxRows || d.NZ + 2 > kLuMaxRows) return EKM_ERR_UNSUPPORTED;
-  size_t npre = 0, nly = 0, nlz = 0, nys = 0, nzs = 0;
+  size_t nly = 0, nlz = 0, nys = 0, nzs = 0;
   bool plain = false, les = false;
   for (int f = 0; f < nf; ++f) {
     if (hf[f].nut) {
@@ -1534,14 +1506,11 @@ int launch_adi_batch(const Dims& d, const Metrics& M, const AdiField* fs, const 
     }
     const Ranges& r = hf[f].r;
     const size_t nk = (size_t)(r.ze - r.zs + 1), nj = (size_t)(r.je - r.js + 1);
-    npre = std::max(npre, (size_t)d.NX2 * nk * nj);
     nly = std::max(nly, nk);
     nlz = std::max(nlz, nj);
     nys = std::max(nys, (size_t)d.NX2 * nk);
     nzs = std::max(nzs, (size_t)d.NX2 * nj);
   }
-  hipLaunchKernelGGL(k_adi_pre, dim3(nblk(npre, 256), nf), dim3(256), 0, st, d, M, fs, t1);
-  EKM_CHECK(hipGetLastError());
   if (plain) {
     hipLaunchKernelGGL(k_lu, dim3((unsigned)nly, nf), dim3(kLuBlock), 0, st, d, M, fs, t1, 0);
     EKM_CHECK(hipGetLastError());

@@ -983,10 +983,9 @@ static int enqueue_substep(ekm_solver* s, const SubstepPlan& q, bool timed) {
     fb.f[f].rg = v ? s->rv : s->rt;
   }
   TRY(launch_flux_accum(s->fft, d, s->M, fb, s->U[0], s->U2b, s->U3b, s->kx, temp5, st));
-  {
-    double* r[4] = {s->R[0], s->R[1], s->R[2], s->RTH};
-    TRY(fft_inverse_n(s->fft, r, fb.n, (long)d.plane, st));
-  }
+  // R to physical space with the explicit half operators of the implicit solves
+  const AdiT1 t1{s->ss, {1.0, 1.0, 1.0, p.pr}};
+  TRY(launch_inv_pre(s->fft, d, s->M, q.les_on ? s->adi_dl : s->adi_d, s->adi_nf, t1, q.les_on, st));
   // LES_WALL_MODEL (:1687-1691) from the velocities entering the implicit
   // solves, in physical space here as there
   if (q.wall_on) {
@@ -1007,7 +1006,6 @@ static int enqueue_substep(ekm_solver* s, const SubstepPlan& q, bool timed) {
   // implicit solves are independent, so they share one set of launches
   {
     const int corners = th ? ((p.th_bc[EKM_ZMAX] == 1 ? 1 : 0) | (p.th_bc[EKM_ZMIN] == 6 ? 2 : 0)) : 0;
-    AdiT1 t1{s->ss, {1.0, 1.0, 1.0, p.pr}};
     TRY(launch_adi_batch(d, s->M, q.les_on ? s->adi_dl : s->adi_d, q.les_on ? s->adi_hl : s->adi_h, s->adi_nf, t1,
                          3, corners, st, s->tn));
   }
