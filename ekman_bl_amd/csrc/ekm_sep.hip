@@ -47,8 +47,10 @@ constexpr double kSepFp64Shift = 6e-5;
 constexpr double kSepPin = 1e20;
 
 constexpr int kCols = 128;   // columns per workgroup of the products: 4 wavefronts of 32
-constexpr int kRowsUpd = 2;  // points per thread of the residual update
-constexpr int kSolvesUpd = 8;  // solves per workgroup of the residual update
+// Residual passes: points per thread and solves per workgroup, by pick_upd.
+struct UpdSplit {
+  int rows, solves;
+};
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -339,10 +341,12 @@ __device__ inline void wave_max_to(unsigned long long* to, double v) {
 
 // per-solve state, and the rows of z without an unknown (the products leave
 // them out): zero
-__global__ void __launch_bounds__(256) k_sep_clear(unsigned long long* rm, int n, int* cycles, int ns, float* z, int nx,
-                                                   int ny, int j0, int nk) {
+// (open: the solves start without a look at their right-hand sides, so the
+// first pass finds them unsolved)
+__global__ void __launch_bounds__(256) k_sep_clear(unsigned long long* rm, int n, int nsmax, int open, int* cycles, int ns,
+                                                   float* z, int nx, int ny, int j0, int nk) {
   const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t < n) rm[t] = 0ull;
+  if (t < n) rm[t] = open && t < nsmax ? 0x7ff0000000000000ull : 0ull;
   if (t < ns) cycles[t] = 0;
   const int rows = ny - nk;  // 0..2
   if (t < ns * rows * nx) {
@@ -388,23 +392,23 @@ __device__ inline double stencil(double k0, double k2, double k4, double k6, dou
   return (k0 * (double)xe + k2 * (double)xn) + (k4 * (double)xw + k6 * (double)xs) + k9 * (double)xc;
 }
 
-// The start of every solve: max|b|, and where a later pass needs it (a start
-// from a guess, the singular problem's compatible right-hand side) the
-// residual r = b - guess A phi.  Solves of one workgroup share the coefficients.
-template <bool PER>
+// The start of a solve that does not begin with r = b as it stands (a start from
+// a guess, the singular problem's compatible right-hand side): the residual
+// r = b - guess A phi and its max.
+template <bool PER, int RU>
 __global__ void __launch_bounds__(256) k_sep_start(SepStencil S, int nsolve, const double* __restrict__ guessp,
                                                    const double* __restrict__ rhs, const double* __restrict__ phi,
-                                                   const double* __restrict__ wb, int pin, int store,
+                                                   const double* __restrict__ wb, int pin, int su,
                                                    double* __restrict__ r, unsigned long long* __restrict__ rm) {
   const double g = guessp ? *guessp : 0.0;
-  const int p0 = blockIdx.x * (256 * kRowsUpd) + threadIdx.x;
-  const int s0 = blockIdx.y * kSolvesUpd, s1 = min(s0 + kSolvesUpd, nsolve);
+  const int p0 = blockIdx.x * (256 * RU) + threadIdx.x;
+  const int s0 = blockIdx.y * su, s1 = min(s0 + su, nsolve);
   for (int s = s0; s < s1; ++s) {
     const double* rt = rhs + (size_t)s * S.n;
     const double* ph = phi + (size_t)s * S.n;
     double mx = 0.0;
 #pragma unroll
-    for (int u = 0; u < kRowsUpd; ++u) {
+    for (int u = 0; u < RU; ++u) {
       const int p = p0 + 256 * u;
       if (p >= S.n) continue;
       const bool sp = S.spec[p];
@@ -421,7 +425,7 @@ __global__ void __launch_bounds__(256) k_sep_start(SepStencil S, int nsolve, con
         v -= g * ((S.c[p] * xe + S.c[2 * (size_t)S.n + p] * xn) +
                   (S.c[4 * (size_t)S.n + p] * xw + S.c[6 * (size_t)S.n + p] * xs) + k9 * ph[p]);
       }
-      if (store) r[(size_t)s * S.n + p] = v;
+      r[(size_t)s * S.n + p] = v;
       mx = fmax(mx, fabs(v));
     }
     wave_max_to(rm + s, mx);
@@ -431,17 +435,17 @@ __global__ void __launch_bounds__(256) k_sep_start(SepStencil S, int nsolve, con
 // phi += z, r -= A z and max|r| of every solve that has not ended (first pass:
 // phi = guess*phi + z; from a zero start r is b, read from the right-hand
 // sides).  Bound by memory: 36 bytes per point and solve (28 in the first
-// pass); the coefficients are read once for kSolvesUpd solves.
-template <bool PER>
+// pass).
+template <bool PER, int RU>
 __global__ void __launch_bounds__(256) k_sep_update(SepStencil S, int nsolve, int first, int from_rhs, int it,
                                                     const double* __restrict__ guessp,
                                                     const double* __restrict__ rhs, const float* __restrict__ z,
                                                     double* __restrict__ r, double* __restrict__ phi,
                                                     const unsigned long long* __restrict__ rm,
                                                     unsigned long long* __restrict__ rm_next, double tol,
-                                                    int* __restrict__ cycles) {
-  const int p0 = blockIdx.x * (256 * kRowsUpd) + threadIdx.x;
-  const int s0 = blockIdx.y * kSolvesUpd, s1 = min(s0 + kSolvesUpd, nsolve);
+                                                    int* __restrict__ cycles, int su) {
+  const int p0 = blockIdx.x * (256 * RU) + threadIdx.x;
+  const int s0 = blockIdx.y * su, s1 = min(s0 + su, nsolve);
   const double g = (first && guessp) ? *guessp : 0.0;
   if (blockIdx.x == 0 && threadIdx.x < s1 - s0) {
     const int s = s0 + threadIdx.x;
@@ -450,11 +454,11 @@ __global__ void __launch_bounds__(256) k_sep_update(SepStencil S, int nsolve, in
     else
       cycles[s] = it;
   }
-  int i[kRowsUpd], j[kRowsUpd], pp[kRowsUpd];
-  bool in[kRowsUpd], sp[kRowsUpd];
-  double k0[kRowsUpd], k2[kRowsUpd], k4[kRowsUpd], k6[kRowsUpd], kb[kRowsUpd], kj[kRowsUpd];
+  int i[RU], j[RU], pp[RU];
+  bool in[RU], sp[RU];
+  double k0[RU], k2[RU], k4[RU], k6[RU], kb[RU], kj[RU];
 #pragma unroll
-  for (int u = 0; u < kRowsUpd; ++u) {
+  for (int u = 0; u < RU; ++u) {
     const int p = p0 + 256 * u;
     in[u] = p < S.n;
     const int q = in[u] ? p : S.n - 1;
@@ -474,26 +478,30 @@ __global__ void __launch_bounds__(256) k_sep_update(SepStencil S, int nsolve, in
     if (solved(rm, s, tol)) {
       // a solve that met the tolerance at its start takes the scaled guess
       if (first)
-        for (int u = 0; u < kRowsUpd; ++u)
+        for (int u = 0; u < RU; ++u)
           if (in[u]) phi[o + pp[u]] = (g != 0.0 && !sp[u]) ? g * phi[o + pp[u]] : 0.0;
       continue;
     }
     const double kx2 = S.kx2[s >> 1];
-    double mx = 0.0;
+    double mx = 0.0, rv[RU], ph[RU], az[RU], zc[RU];
 #pragma unroll
-    for (int u = 0; u < kRowsUpd; ++u) {
+    for (int u = 0; u < RU; ++u) {
       const int p = pp[u];
-      const double az = stencil<PER>(k0[u], k2[u], k4[u], k6[u], kb[u] - kx2 * kj[u], z + o, p, i[u], j[u], S.nx, S.ny);
-      const double rv = from_rhs ? (sp[u] ? 0.0 : -rhs[o + p]) : r[o + p];
-      double ph = 0.0;
-      if (!first)
-        ph = phi[o + p];
-      else if (g != 0.0 && !sp[u])
-        ph = g * phi[o + p];
-      const double rn = rv - az, pn = ph + (double)z[o + p];
+      rv[u] = from_rhs ? -rhs[o + p] : r[o + p];
+      ph[u] = (!first || g != 0.0) ? phi[o + p] : 0.0;
+      zc[u] = (double)z[o + p];
+      az[u] = stencil<PER>(k0[u], k2[u], k4[u], k6[u], kb[u] - kx2 * kj[u], z + o, p, i[u], j[u], S.nx, S.ny);
+    }
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      if (first) {
+        if (from_rhs && sp[u]) rv[u] = 0.0;
+        ph[u] = sp[u] ? 0.0 : g * ph[u];
+      }
+      const double rn = rv[u] - az[u];
       if (in[u]) {
-        r[o + p] = rn;
-        phi[o + p] = pn;
+        r[o + pp[u]] = rn;
+        phi[o + pp[u]] = ph[u] + zc[u];
         mx = fmax(mx, fabs(rn));
       }
     }
@@ -810,6 +818,20 @@ int launch_lines(int nx, int nk, int m0, int nm, const T* fac, float* t, long ld
   return EKM_OK;
 }
 
+// A thread's loads of all its points are in flight together, and its points'
+// coefficients serve all solves of its workgroup: as many of both as leave the
+// chip 4 workgroups per compute unit (1024), below which it stands partly idle.
+// Together with the zero start that reads no right-hand side, per step against
+// 2 points and 8 solves for every size: 256x385x769 with both subgrid models
+// 123.9 -> 118.4 ms, 512x257x513 60.5 -> 58.6, 256x193x257 12.44 -> 12.00,
+// 64x65x65 from graphs 1.288 -> 1.220.
+UpdSplit pick_upd(int n, int nsolve) {
+  for (int rows = 4; rows > 1; rows >>= 1)
+    for (int solves = 8; solves > 1; solves >>= 1)
+      if ((long)((n + 256 * rows - 1) / (256 * rows)) * ((nsolve + solves - 1) / solves) >= 1024) return {rows, solves};
+  return {1, 2};
+}
+
 template <bool PER>
 int solve_typed(const SepPlan& sp, const SepBuffers& b, int nsolve, const double* guess, hipStream_t st) {
   const int nx = sp.nx, ny = sp.ny, nk = sp.nk, nmode = (nsolve + 1) / 2;
@@ -818,15 +840,26 @@ int solve_typed(const SepPlan& sp, const SepBuffers& b, int nsolve, const double
   const SepStencil S{b.cf64, sp.base, b.spec, sp.kx2, nx, ny, n};
   float *t1 = b.t, *t2 = b.t + (size_t)nsolve * n;
   unsigned long long* rm = sp.rmax;
-  const int ncl = std::max(std::max((K + 1) * nm, nsolve), nsolve * (ny - nk) * nx);
-  hipLaunchKernelGGL(k_sep_clear, dim3((unsigned)((ncl + 255) / 256)), dim3(256), 0, st, rm, (K + 1) * nm, b.cycles, nsolve,
-                     t2, nx, ny, sp.j0, nk);
   const bool sing = b.wnull != nullptr;
-  if (sing) hipLaunchKernelGGL(k_sep_null, dim3(2), dim3(1024), 0, st, b.wnull, b.rhs, b.spec, n, sp.wb);
-  const dim3 gu((unsigned)((n + 256 * kRowsUpd - 1) / (256 * kRowsUpd)), (unsigned)((nsolve + kSolvesUpd - 1) / kSolvesUpd));
+  // r = b as it stands is read from the right-hand sides by the first pass
   const int store = guess != nullptr || sing;
-  hipLaunchKernelGGL((k_sep_start<PER>), gu, dim3(256), 0, st, S, nsolve, guess, b.rhs, b.phi, sing ? sp.wb : nullptr, sp.pin,
-                     store, b.r, rm);
+  const int ncl = std::max(std::max((K + 1) * nm, nsolve), nsolve * (ny - nk) * nx);
+  hipLaunchKernelGGL(k_sep_clear, dim3((unsigned)((ncl + 255) / 256)), dim3(256), 0, st, rm, (K + 1) * nm, nm, !store,
+                     b.cycles, nsolve, t2, nx, ny, sp.j0, nk);
+  if (sing) hipLaunchKernelGGL(k_sep_null, dim3(2), dim3(1024), 0, st, b.wnull, b.rhs, b.spec, n, sp.wb);
+  const UpdSplit us = pick_upd(n, nsolve);
+  const unsigned gy = (unsigned)((nsolve + us.solves - 1) / us.solves);
+  EKM_CHECK(hipGetLastError());
+  const dim3 gu((unsigned)((n + 256 * us.rows - 1) / (256 * us.rows)), gy);
+#define START(RU)                                                                                                 \
+  hipLaunchKernelGGL((k_sep_start<PER, RU>), gu, dim3(256), 0, st, S, nsolve, guess, b.rhs, b.phi,                \
+                     sing ? sp.wb : nullptr, sp.pin, us.solves, b.r, rm)
+  if (store) {
+    if (us.rows == 4) START(4);
+    else if (us.rows == 2) START(2);
+    else START(1);
+  }
+#undef START
   EKM_CHECK(hipGetLastError());
   for (int it = 1; it <= K; ++it) {
     const unsigned long long* rp = rm + (size_t)(it - 1) * nm;
@@ -843,8 +876,13 @@ int solve_typed(const SepPlan& sp, const SepBuffers& b, int nsolve, const double
     if (e != EKM_OK) return e;
     e = launch_gemm<float>(sp.mt, sp.ab, nk, nx, nsolve, n, t1, 1.f, t2 + jo, rp, b.tol, st);
     if (e != EKM_OK) return e;
-    hipLaunchKernelGGL((k_sep_update<PER>), gu, dim3(256), 0, st, S, nsolve, (int)first, from_rhs, it, guess, b.rhs, t2, b.r,
-                       b.phi, rp, rm + (size_t)it * nm, b.tol, b.cycles);
+#define UPD(RU)                                                                                                        \
+  hipLaunchKernelGGL((k_sep_update<PER, RU>), gu, dim3(256), 0, st, S, nsolve, (int)first, from_rhs, it, guess, b.rhs, t2, \
+                     b.r, b.phi, rp, rm + (size_t)it * nm, b.tol, b.cycles, us.solves)
+    if (us.rows == 4) UPD(4);
+    else if (us.rows == 2) UPD(2);
+    else UPD(1);
+#undef UPD
     EKM_CHECK(hipGetLastError());
   }
   if (sing) hipLaunchKernelGGL(k_sep_shift, dim3(2), dim3(1024), 0, st, b.phi, n, sp.pin);

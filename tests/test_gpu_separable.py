@@ -84,3 +84,28 @@ def test_repeated_solves_are_identical():
     a, _ = _run(p, xp, yp, ic, 2)
     b, _ = _run(p, xp, yp, ic, 2)
     assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("nx,ny2,nz2,bcs", [
+    (128, 97, 129, (2, 2, 2, 1)),     # two points per thread and a remainder
+    (128, 129, 193, (2, 2, 2, 1)),    # four points per thread and a remainder
+    (128, 129, 193, (2, 2, 2, 2)),    # singular kx = 0: the start's residual is stored
+])
+def test_residual_pass_splits(nx, ny2, nz2, bcs):
+    """The residual pass with several points per thread, from a zero start and
+    from a guess, within the bounds of the comparison above."""
+    cfg = config(1)
+    p = cfg.params
+    p.nx, p.ny, p.nz = nx, ny2 - 2, nz2 - 2
+    p.mg_ixp, p.mg_iex = mg_factors(nz2)
+    p.mg_jyq, p.mg_jey = mg_factors(ny2)
+    p.delta_t = 0.02
+    for k, b in enumerate(bcs):
+        p.mudpack_bc[k] = b
+    xp, yp = tanh_grid(p.ny, p.nz, p.ly, p.lz, cfg.gamma)
+    ic = ekman_initial(p, yp, 3, 0.05, 0.0)
+    ref, _ = _run(p, xp, yp, ic, 1)
+    for guess in (0, 1):
+        got, cyc = _run(p, xp, yp, ic, 2, guess)
+        r = [_rel(a, b) for a, b in zip(got[:4], ref[:4])]
+        assert max(r[:3]) < 1e-8 and r[3] < 1e-6 and cyc.max() <= 5
