@@ -258,6 +258,18 @@ __device__ inline double bc_rhs(const Dims& d, const Metrics& M, const BcRow& e,
   }
 }
 
+// The y sweep's solution on rows JSTART..JEND is not needed in memory (the sweep
+// itself forms the z right-hand side from it, and the z sweep rewrites those
+// rows whole) unless a lagged z row reads column K of it.
+// Without that store (8 of the sweep's 48 bytes per point) a step of 256x385x769
+// with both subgrid models takes 121.8 instead of 123.5 ms, 256x193x257 in the
+// plain form 51.42 instead of 51.75 (runs of one build within 0.3%).
+__device__ inline bool z_lag_source(const BcTable& bz, int K) {
+  bool k = false;
+  for (int e = 0; e < 4; ++e) k = k || (bz.r[e].kind == BC_LAGGED && bz.r[e].src == K);
+  return k;
+}
+
 // y sweep for lines (i,K): solves in place into U, then emits the z-sweep
 // right-hand side R = S/2 + J U* + t1 [G22(J+1)(U*(J+1)-U*) - G22(J)(U*-U*(J-1))]
 // (:1460-1478 for theta, :1744-1757 for U1, ...).
@@ -329,6 +341,7 @@ __global__ void __launch_bounds__(256) k_ysweep(Dims d, Metrics M, const AdiFiel
       U[q0 + dj * row] = g;
     }
   }
+  const bool keep = z_lag_source(F.bz, K);
   double x2 = 0.0, x1 = g / piv[base + N];  // x1 = x(row+1), x2 = x(row+2)
   U[q0 + dj * N] = x1;
   for (int row0 = N - 1; row0 >= 0; row0 -= kSw) {
@@ -351,7 +364,7 @@ __global__ void __launch_bounds__(256) k_ysweep(Dims d, Metrics M, const AdiFiel
       const int row = row0 - u;
       if (row < 0) break;
       const double x0 = (gg[u] - uu[u] * x1) / pp[u];
-      U[q0 + dj * row] = x0;
+      if (keep || row < r.js || row > r.je) U[q0 + dj * row] = x0;
       const int jr = row + 1;  // R at row+1 now has x(row), x(row+1), x(row+2)
       if (jr >= r.js && jr <= r.je)
         R[q0 + dj * jr] = 0.5 * ss[u] + jc[u] * x1 + t1 * (gp[u] * (x2 - x1) - g0[u] * (x1 - x0));
@@ -539,6 +552,7 @@ __global__ void __launch_bounds__(256) k_ysweep_les(Dims d, Metrics M, const Adi
       nc = np;
     }
   }
+  const bool keep = z_lag_source(F.bz, K);
   double x2 = 0.0, x1 = g / pvp;  // x1 = x(row+1), x2 = x(row+2)
   U[q0 + dj * N] = x1;
   double n1 = nut[q0 + dj * N], n2 = 0.0;  // NU_T at row+1, row+2
@@ -581,7 +595,7 @@ __global__ void __launch_bounds__(256) k_ysweep_les(Dims d, Metrics M, const Adi
       for (int e = 0; e < 4; ++e)
         if (bc.r[e].row == row) c = bc.r[e].c;
       const double x0 = (gg[u] - c * x1) / pp[u];
-      U[q0 + dj * row] = x0;
+      if (keep || row < r.js || row > r.je) U[q0 + dj * row] = x0;
       const int jr = row + 1;  // R at row+1 now has x(row), x(row+1), x(row+2)
       if (jr >= r.js && jr <= r.je) {
         double rv = 0.5 * ss[u] + jc[u] * x1 + t1 * (gp[u] * (x2 - x1) - g0[u] * (x1 - x0));
