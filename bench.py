@@ -12,11 +12,11 @@ flow, on which the reference does not run the subgrid models, so the models
 run in every timed step.
 
 Forms (each from the same seeded state, each checked against the bound):
-- headline (`value`): the consistent projection with FP32 alternating-line
-  V(1,1) cycles inside FP64 GCR(1) outer iterations (proj_mode 2, max|residual|
-  <= 1e-12 per real solve), all solves of a projection and all ADI systems of
-  a substep batched; launched eagerly so that the projection's solve kernel is
-  timed with HIP events on the solver's stream (`roofline`);
+- headline (`value`): the consistent projection with FP32 separable solves of
+  the planes inside FP64 residual iterations (proj_mode 2 on a rectilinear grid,
+  max|residual| <= 1e-12 per real solve), all solves of a projection and all ADI
+  systems of a substep batched; launched eagerly so that the projection's solve
+  kernels are timed with HIP events on the solver's stream (`roofline`);
 - the same replayed from captured HIP graphs (`forms.graph`);
 - the same started from the learned guess (`forms.learned`, when trained
   weights are found);
@@ -57,7 +57,8 @@ HBM_PEAK_GBS = 8000.0
 DIV_BOUND = 1e-10
 FORM_NAMES = {0: "plain FP64 MUDPACK-replica W(2,1), relmax 1e-6",
               1: "consistent projection, FP64 alternating-line V(1,1)",
-              2: "consistent projection, FP32 alternating-line V(1,1) cycles in FP64 outer iterations"}
+              2: "consistent projection, FP32 separable solves in FP64 residual iterations"}
+CYCLE_TYPES = {0: "W(2,1) point GS", 1: "V(1,1) alternating zebra line GS", 2: "separable solve of the plane"}
 DATA = os.path.join(ROOT, "ekman_bl_amd", "data")
 
 
@@ -126,7 +127,7 @@ def workload_name(cfg, mode: int, tol: float, krylov: int) -> str:
             + (", dynamic Smagorinsky LES of velocity and scalar" if cfg.params.les_model else "")
             + f", {FORM_NAMES[mode]}"
             + (f", max|residual| <= {tol:g}" if mode else "")
-            + (", GCR(1) outer iteration" if mode and krylov else ""))
+            + (", GCR(1) outer iteration" if mode == 1 and krylov else ""))
 
 
 def traffic_file(cfg) -> str:
@@ -291,10 +292,13 @@ def main() -> int:
         cbar = h["cycles"] / max(h["solves"], 1)
         launch_bytes = roofline.mg_launch_bytes(p, nsolve, cbar)
         kname = "k_mg_solve (batched MUDPACK replica, one launch per projection)"
-    else:
-        width = 4 if args.mode == 2 else 8
-        launch_bytes = roofline.tight_launch_bytes(p, nsolve, cyc_per_launch, width, args.krylov)
+    elif args.mode == 1:
+        launch_bytes = roofline.tight_launch_bytes(p, nsolve, cyc_per_launch, 8, args.krylov)
         kname = "k_tight_solve (batched consistent projection, one launch per projection)"
+    else:  # the configurations' grids are rectilinear: the separable solver takes them
+        launch_bytes = roofline.sep_launch_bytes(p, nsolve, cyc_per_launch)
+        kname = "k_sep_* (separable consistent projection, the launches of one projection together)"
+    launch_flops = roofline.sep_launch_flops(p, cyc_per_launch) if args.mode == 2 else None
     achieved = launch_bytes / (avg_ms * 1e-3) / 1e9
     log(f"[bench] {ms_per_step:.2f} ms/step, {value:.1f} Mpt-steps/s, solve {avg_ms:.3f} ms/launch, "
         f"cycles/step {h['cyc'] / args.steps:.0f}, div_max {h['div_max']:.3e}")
@@ -319,30 +323,30 @@ def main() -> int:
     ref_state = None
     if args.side_steps > 0:
         sw, ss = args.side_warmup, args.side_steps
-        vc = "V(1,1) alternating zebra line GS"
+        vc, sc = CYCLE_TYPES[1], CYCLE_TYPES[2]
         log(f"[bench] form 1 ({FORM_NAMES[1]}): {sw} + {ss} steps")
         r1 = run_form(cfg, xp, yp, ic, 1, ss, sw, args.tol, args.krylov, keep_state=True)
         ref_state = r1.pop("state")
         add_form("fp64_cycles", r1, FORM_NAMES[1] + ", GCR(1)", vc)
-        for key, kw, desc in (("fp32_cycles", {}, FORM_NAMES[2] + ", GCR(1)"),
-                              ("graph", {"graph": True}, FORM_NAMES[2] + ", GCR(1), substeps replayed from HIP graphs")):
+        for key, kw, desc in (("fp32_cycles", {}, FORM_NAMES[2]),
+                              ("graph", {"graph": True}, FORM_NAMES[2] + ", substeps replayed from HIP graphs")):
             log(f"[bench] {key}: {sw} + {ss} steps")
             r = run_form(cfg, xp, yp, ic, 2, ss, sw, args.tol, args.krylov, keep_state=True, **kw)
-            add_form(key, r, desc, vc, ref_state)
+            add_form(key, r, desc, sc, ref_state)
             del r
             gc.collect()
         net, src = learned_net(p, args.learned)
         if net is not None:
             log(f"[bench] learned start ({src}): {sw} + {ss} steps")
             r = run_form(cfg, xp, yp, ic, 2, ss, sw, args.tol, args.krylov, net=net, keep_state=True)
-            add_form("learned", r, FORM_NAMES[2] + f", GCR(1), solves started from the learned guess ({src})", vc,
+            add_form("learned", r, FORM_NAMES[2] + f", solves started from the learned guess ({src})", sc,
                      ref_state)
             del r
             net.close()
             gc.collect()
         log(f"[bench] form 0 ({FORM_NAMES[0]}): {sw} + {ss} steps")
         r0 = run_form(cfg, xp, yp, ic, 0, ss, sw, args.tol, args.krylov, keep_state=True)
-        add_form("plain_fp64_mudpack", r0, FORM_NAMES[0], "W(2,1) point GS", ref_state)
+        add_form("plain_fp64_mudpack", r0, FORM_NAMES[0], CYCLE_TYPES[0], ref_state)
         del r0
         gc.collect()
     workload = workload_name(cfg, args.mode, args.tol, args.krylov)
@@ -366,7 +370,7 @@ def main() -> int:
         "div_max_max": h["div_max"],
         "meets_div_bound": bool(h["div_max"] < DIV_BOUND),
         "mg_cycles_per_step": round(h["cyc"] / args.steps, 2),
-        "cycle_type": "V(1,1) alternating zebra line GS" if args.mode else "W(2,1) point GS",
+        "cycle_type": CYCLE_TYPES[args.mode],
         "dt_final": h["dt"],
         "speedup_vs_fp64_cycles": round(fp64["ms_per_step"] / ms_per_step, 3) if fp64 else None,
         "speedup_vs_plain_fp64_mudpack": (round(forms["plain_fp64_mudpack"]["ms_per_step"] / ms_per_step, 3)
@@ -377,7 +381,9 @@ def main() -> int:
                      "traffic_cycles_per_launch": tr[1] if tr else None,
                      "traffic_source": tr[2] if tr else None,
                      "avg_launch_ms": round(avg_ms, 4), "cycles_per_launch": round(cyc_per_launch, 1),
-                     "algorithmic_bytes_per_launch": int(launch_bytes)},
+                     "algorithmic_bytes_per_launch": int(launch_bytes),
+                     "matrix_f32_tflops": round(launch_flops / (avg_ms * 1e-3) / 1e12, 2) if launch_flops else None,
+                     "matrix_f32_peak_tflops": 157.3 if launch_flops else None},
         "forms": forms,
         "tuning": tuning_of(cfg, args.mode),
     }

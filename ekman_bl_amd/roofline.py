@@ -83,3 +83,31 @@ def tight_step_bytes(p, cycles_per_projection: float, width: int, krylov: int = 
     npts = p.nx * (p.ny + 2) * (p.nz + 2)
     nsolve = 2 * (p.nx // 3 + 1)
     return 8.0 * npts * (34 * F + 33) + 3 * tight_launch_bytes(p, nsolve, cycles_per_projection, width, krylov)
+
+
+# ---------------------------------------------------------------------------
+# The separable solve of the consistent projection (proj_mode 2 on a grid
+# without cross terms), per pass, real solve and plane point: the forward product
+# reads the FP64 residual (or right-hand side) and writes FP32 (12), the z lines
+# read and write it (8) and read three FP32 factors shared by the two solves of a
+# mode (6), the product back reads and writes FP32 (8), and the residual update
+# reads the correction, r and phi and writes r and phi (36; a first pass from a
+# zero start reads no phi: 28).  The matrices and the stencil are shared by all
+# solves and not counted.  Each product is 2 flops per eigenmode and point.
+# ---------------------------------------------------------------------------
+SEP_PASS = 70.0
+
+
+def sep_rows(p) -> int:
+    """Rows of a plane that hold unknowns (specified y ends do not)."""
+    return p.ny + 2 - (p.mudpack_bc[2] == 1) - (p.mudpack_bc[3] == 1)
+
+
+def sep_launch_bytes(p, nsolve: int, passes_total: float) -> float:
+    """Algorithmic bytes of one projection (all solves; passes summed over them)."""
+    return (p.ny + 2) * (p.nz + 2) * (SEP_PASS * passes_total - 8.0 * min(nsolve, passes_total))
+
+
+def sep_launch_flops(p, passes_total: float) -> float:
+    """FP32 matrix operations of one projection."""
+    return 4.0 * sep_rows(p) ** 2 * (p.nz + 2) * passes_total
