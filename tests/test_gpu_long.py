@@ -3,7 +3,7 @@
 - the plain FP64 form (MUDPACK replica) over all 100 steps of the 64x65x65
   neutral case, and over 10 steps of the 256x193x257 stratified case, held to
   1e-10 relative L2 per field with the relative error printed every few steps;
-- the headline form (FP32 cycles inside FP64 residual iterations, GCR(1),
+- the headline form (FP32 solves inside FP64 residual iterations,
   max|residual| <= 1e-12) over all 100 steps of the 64x65x65 case against the
   oracle's FP64 consistent projection, per field, at <= 1e-8 (the pressure,
   which sums phi / H_BAR over the substeps, at <= 1e-6), and its distance

@@ -186,9 +186,11 @@ def test_step_matches_oracle(n, steps, oracle_lib):
 
 @pytest.mark.parametrize("mode,n,krylov", [(1, 1, 0), (2, 1, 0), (1, 2, 0), (2, 2, 0), (2, 1, 1), (2, 2, 1), (1, 2, 1)])
 def test_consistent_projection_matches_oracle(mode, n, krylov, oracle_lib):
-    """proj_mode 1 (FP64 line multigrid) and 2 (FP32 cycles inside FP64
-    residual iterations), with the plain or the GCR(1) outer iteration,
-    against the oracle's FP64 consistent solve:
+    """proj_mode 1 (FP64 line multigrid) and 2 (FP32 solves inside FP64 residual
+    iterations; separable ones on these grids, so that proj_krylov has no
+    effect there), with the plain or the GCR(1) outer iteration, against the
+    oracle's FP64 consistent solve (mode 2's V cycles without cross terms:
+    test_gpu_separable.py):
     all converge to the same discrete solution, so the fields agree to the
     solve tolerance (relative L2 <= 5e-9 for mode 1, <= 1e-8 for mode 2, at
     max|residual| <= 1e-12), and the divergence after the projection is below
@@ -229,8 +231,9 @@ def test_consistent_projection_periodic_ends_match_oracle(top, mode, krylov, ske
     with phi = 0 at (K = 0, J = NY+1) that satisfies every other row, which
     the oracle pins and the GPU reaches through a compatible right-hand side);
     `skew` shears the grid so that the cross terms, which read the periodic
-    virtual columns diagonally, are active.  A full step of the small stratified case, FP64 and
-    FP32 cycles, against the oracle's FP64 consistent solve: velocities and
+    virtual columns diagonally, are active.  A full step of the small stratified case, FP64
+    cycles and FP32 solves (V cycles on the sheared grid, separable solves on the others),
+    against the oracle's FP64 consistent solve: velocities and
     scalar to 1e-8 relative L2, the pressure (which sums phi / H_BAR over the
     substeps) to 1e-6, divergence below 1e-10, every solve converged."""
     from ekman_bl_amd.params import YMAX, YMIN, ZMIN, ZMAX

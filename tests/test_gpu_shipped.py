@@ -9,7 +9,7 @@ velocity scale (WBULK0 = 0.05) with 5% noise (the run's DIABLO.START is not
 shipped), and the background scalar a stable linear profile (the run reads
 TH_BAR from its restart).
 
-The consistent projection (FP32 cycles, GCR(1)) must hold max |J div u|
+The consistent projection (FP32 solves) must hold max |J div u|
 below 1e-10 after the initial projection and every substep of two steps,
 with every solve converged, the singular kx = 0 solve included (its
 right-hand side made compatible with the operator's left null vector); the
