@@ -1,8 +1,9 @@
 """The kernel tuning (ekm_tuning) changes launch geometry and memory
 placement only: every allowed value of every parameter gives the same state
 bit for bit, on a stratified case with both subgrid models and the headline
-projection form, and on the 64x65x65 case with the MUDPACK replica.  The
-autotuner's search returns one of those tunings."""
+projection form (rectilinear, and sheared, where its V cycles run), and on the
+64x65x65 case with the MUDPACK replica.  The autotuner's search returns one of
+those tunings."""
 import numpy as np
 import pytest
 
@@ -16,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _case(name):
-    if name == "les_fp32":
+    if name != "replica":
         cfg = config(2)
         p = cfg.params
         p.nx, p.ny, p.nz = 32, 31, 31
@@ -28,6 +29,8 @@ def _case(name):
         p = cfg.params
         p.proj_mode = 0
     xp, yp = tanh_grid(p.ny, p.nz, p.ly, p.lz, cfg.gamma)
+    if name == "les_fp32_sheared":
+        xp = xp + 0.05 * np.sin(0.3 * yp)
     return p, xp, yp, ekman_initial(p, yp, cfg.seed, cfg.noise, cfg.th_noise)
 
 
@@ -41,7 +44,7 @@ def _run(p, xp, yp, ic, tuning):
     return out, got
 
 
-@pytest.mark.parametrize("name", ["les_fp32", "replica"])
+@pytest.mark.parametrize("name", ["les_fp32", "les_fp32_sheared", "replica"])
 def test_every_tuning_gives_the_same_state(name):
     p, xp, yp, ic = _case(name)
     ref, t0 = _run(p, xp, yp, ic, None)
