@@ -43,16 +43,30 @@ def test_replica_matches_oracle(ny2, nz2, bcs, oracle_lib):
     for q in range(len(kx2)):
         po, co = o.mudpack(kx2[q], rhs[q])
         print(f"[5-point {ny2}x{nz2} {bcs}] kx2 {kx2[q]}: cycles {cyc[q]}/{co} rel {_rel(phi[q], po):.1e}", flush=True)
-        assert cyc[q] == co and _rel(phi[q], po) < 1e-12
-    # a given start: two calls of iguess = 1 agree, and lower the residual's change
+        assert cyc[q] == co and np.array_equal(phi[q], po)
+    s.close()
+    # a given start (iguess = 1): 6 cycles from zero and 6 more from their result
+    # are 12 cycles from zero, bit for bit.  With periodic sides the first sweep
+    # of a given start finds zero virtual points, so there the result only lies
+    # near that of the 12 cycles (within half of what the 6 more change).
+    t = p.copy()
+    t.mg_tolmax = 1e-300
+    s = S.DuctSolver(t, xp, yp)
+    start, _ = s.multigrid_mudpack(kx2, rhs)
     L = S.lib()
     L.ekm_multigrid_mudpack_ex.argtypes = [ctypes.c_void_p, ctypes.c_int] + [S._D] * 3 + [ctypes.POINTER(ctypes.c_int),
                                                                                           ctypes.c_int]
-    out = []
-    for _ in range(2):
-        g = phi.copy()
-        c = (ctypes.c_int * len(kx2))()
-        assert L.ekm_multigrid_mudpack_ex(s.h, len(kx2), S._p(kx2), S._p(rhs), S._p(g), c, 1) == 0
-        out.append(g)
-    assert np.array_equal(out[0], out[1]) and np.all(np.isfinite(out[0]))
+    more = start.copy()
+    c = (ctypes.c_int * len(kx2))()
+    assert L.ekm_multigrid_mudpack_ex(s.h, len(kx2), S._p(kx2), S._p(rhs), S._p(more), c, 1) == 0
     s.close()
+    t.mg_maxcy = 12
+    o = oracle_lib.Oracle(t, xp, yp)
+    for q in range(len(kx2)):
+        twelve, _ = o.mudpack(kx2[q], rhs[q])
+        e = [_rel(x[q], twelve) for x in (start, more)]
+        print(f"[5-point {ny2}x{nz2} {bcs}] kx2 {kx2[q]}: from 12 cycles {e[0]:.1e} after 6, {e[1]:.1e} after 6 + 6", flush=True)
+        if 0 in bcs:
+            assert e[1] < 0.5 * e[0]
+        else:
+            assert np.array_equal(more[q], twelve)
