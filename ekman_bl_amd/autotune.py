@@ -8,7 +8,8 @@ tests/test_gpu_autotune.py); only the time per step changes.
 
 Search: coordinate descent from the defaults over the parameters that the
 form uses (the replica's workgroup only for proj_mode 0, the subgrid-model
-sweeps only with les_model), each candidate timed over whole steps of the
+sweeps only with les_model, the LDS cap not where the separable passes of
+proj_mode 2 leave the V cycles nothing to do), each candidate timed over whole steps of the
 workload itself after one warm-up step, repeated `passes` times.  Results
 are cached in a JSON file keyed by the workload and the device name.
 
@@ -83,7 +84,10 @@ def tune(p, xp, yp, ic, steps: int = 2, passes: int = 1, log=print) -> dict:
     best_ms = min(time_candidate(p, xp, yp, ic, best, steps) for _ in range(passes))
     trials.append({"tuning": dict(best), "ms_per_step": round(best_ms, 3)})
     log(f"[autotune] default {best}: {best_ms:.2f} ms/step")
-    for key in relevant(p):
+    keys = relevant(p)
+    if p.proj_mode == 2 and (xp == xp[:1]).all() and (yp == yp[:, :1]).all():
+        keys.remove("tight_lds_kib")
+    for key in keys:
         for val in SPACE[key]:
             if val == best[key]:
                 continue
