@@ -291,7 +291,8 @@ def main() -> int:
     if args.mode == 0:
         cbar = h["cycles"] / max(h["solves"], 1)
         launch_bytes = roofline.mg_launch_bytes(p, nsolve, cbar)
-        kname = "k_mg_solve (batched MUDPACK replica, one launch per projection)"
+        # (on rectilinear grids, which all configurations have)
+        kname = "k_mg5_solve (batched MUDPACK replica, one launch per projection)"
     elif args.mode == 1:
         launch_bytes = roofline.tight_launch_bytes(p, nsolve, cyc_per_launch, 8, args.krylov)
         kname = "k_tight_solve (batched consistent projection, one launch per projection)"

@@ -156,8 +156,7 @@ __global__ void k_contravariant(Dims d, Metrics M, Ranges r, const double* __res
 }
 
 // ---------------------------------------------------------------------------
-// ADI: explicit half before the y sweep (:1334-1371, :1640-1665, ...)
-// S = R - J U;  R = S/2 + J U + t1 [G11(K+1)(U(K+1)-U) - G11(K)(U-U(K-1))]
+// ADI sweeps (their right-hand sides: k_inv_pre, ekm_fft.hip)
 // ---------------------------------------------------------------------------
 
 // Per-line factorisation of one sweep (THOMAS_REAL forward elimination,
@@ -262,8 +261,8 @@ __device__ inline double bc_rhs(const Dims& d, const Metrics& M, const BcRow& e,
 // itself forms the z right-hand side from it, and the z sweep rewrites those
 // rows whole) unless a lagged z row reads column K of it.
 // Without that store (8 of the sweep's 48 bytes per point) a step of 256x385x769
-// with both subgrid models takes 121.8 instead of 123.5 ms, 256x193x257 in the
-// plain form 51.42 instead of 51.75 (runs of one build within 0.3%).
+// with both subgrid models takes 0.986 of the time, 256x193x257 in the plain form
+// 0.994 (both builds in turn on one box, runs of one build within 0.3%).
 __device__ inline bool z_lag_source(const BcTable& bz, int K) {
   bool k = false;
   for (int e = 0; e < 4; ++e) k = k || (bz.r[e].kind == BC_LAGGED && bz.r[e].src == K);

@@ -11,6 +11,9 @@
 // value), and on the levels held in LDS the division by c9 is the correctly
 // rounded quotient from the reciprocal (Markstein's correction steps: with
 // y = 1/c9 rounded and q within one ulp, q + (x - q c9) y rounds correctly).
+// That holds for finite operands whose quotient and products neither overflow
+// nor fall below the normal range; a solve that has overflowed may hold NaN
+// where the division gives an infinity (the sweeps around it turn both to NaN).
 //
 // A solve is bound by the latency of those steps (a W cycle visits level l
 // 2^(ngrid-l) times), so every array is kept in a colour layout, where the

@@ -19,9 +19,11 @@
 // by 20..1000), so the solves of a projection end together after 3 passes and
 // none of them is a chain of one workgroup's memory round trips: 1024x385x769
 // is 684 solves of 4 to 8 V cycles otherwise.  A pass counts as one cycle.
-// Measured per projection against the V cycles: 1024x385x769 17.8 ms instead
-// of 67.6, and per step 256x193x257 14.1 ms instead of 28.3, 64x65x65 from
-// graphs 1.41 ms instead of 3.62.
+// Measured per projection against the V cycles: 1024x385x769 12.0 ms instead
+// of 68.8, 256x193x257 0.50 instead of 4.95.  Against a solve to 2e-14, a step
+// that stops at 1e-12 is 4 to 200 times closer in every field than with V cycles
+// (64x65x65 to 256x193x257, and a periodic singular set): the passes end further
+// below the tolerance, and leave less of the smooth error.
 //
 // The decomposition is tried at set-up (sep_plan_build) and used where every
 // coefficient lies within kSepDev of the separable operator's; what has not
@@ -36,8 +38,13 @@
 
 namespace {
 
-// A pass reduces the residual by about the largest relative deviation; 0.02
-// keeps it at least as fast as the V(1,1) cycle's worst rate (about 1/20).
+// A pass reduces the residual by about the largest relative deviation.  The rows
+// of both operators sum to zero without the kx^2 term, so a deviation acts on
+// differences of neighbours only and is not amplified on smooth modes: passes in
+// FP64 on sine, geometric, jumping and noisy spacings, 33 to 769 columns, every
+// kind of sides and kx = 0, reduce max|r| by 0.4 to 1.1 times the deviation each
+// (the first, by up to 14 times it).  0.02 keeps a pass at least as fast as the
+// V(1,1) cycle's worst rate (about 1/20).
 constexpr double kSepDev = 0.02;
 // Lines whose shift lambda_k - kx^2 is below this fraction of the z operator's
 // diagonal are solved in FP64: the rounding of an FP32 factor (6e-8 of the
@@ -518,8 +525,9 @@ __global__ void __launch_bounds__(1024) k_sep_shift(double* __restrict__ phi, in
 }
 
 // Eigenvalues and eigenvectors of the symmetric tridiagonal matrix (d, e):
-// implicit QL iterations with Wilkinson's shift, the rotations accumulated on
-// the rows of zt (zt[k] is the eigenvector of d[k] on exit).
+// the implicit QL method with Wilkinson's shift of Martin and Wilkinson (1968;
+// EISPACK's imtql2, with its recovery where a rotation vanishes), the rotations
+// accumulated on the rows of zt (zt[k] is the eigenvector of d[k] on exit).
 bool tridiag_eigen(std::vector<double>& d, std::vector<double> e, std::vector<double>& zt) {
   const int n = (int)d.size();
   zt.assign((size_t)n * n, 0.0);
@@ -821,10 +829,10 @@ int launch_lines(int nx, int nk, int m0, int nm, const T* fac, float* t, long ld
 // A thread's loads of all its points are in flight together, and its points'
 // coefficients serve all solves of its workgroup: as many of both as leave the
 // chip 4 workgroups per compute unit (1024), below which it stands partly idle.
-// Together with the zero start that reads no right-hand side, per step against
-// 2 points and 8 solves for every size: 256x385x769 with both subgrid models
-// 123.9 -> 118.4 ms, 512x257x513 60.5 -> 58.6, 256x193x257 12.44 -> 12.00,
-// 64x65x65 from graphs 1.288 -> 1.220.
+// Together with the first pass that takes a zero start's residual from the
+// right-hand sides, a step takes this much of its time with 2 points and 8 solves
+// for every size (both builds in turn on one box): 256x385x769 with both subgrid
+// models 0.956, 512x257x513 0.969, 256x193x257 0.965, 64x65x65 from graphs 0.947.
 UpdSplit pick_upd(int n, int nsolve) {
   for (int rows = 4; rows > 1; rows >>= 1)
     for (int solves = 8; solves > 1; solves >>= 1)

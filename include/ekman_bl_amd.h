@@ -87,14 +87,17 @@ typedef struct ekm_params {
    *     returns the solution with phi = 0 at (K = 0, J = NY+1) that satisfies
    *     every other row (its left null vector is computed once at creation) */
   int proj_mode;
-  int proj_maxit;          /* cycle cap of proj_mode 1, 2 */
+  int proj_maxit;          /* cycle cap of proj_mode 1, 2 (a separable pass counts as a cycle) */
   double proj_tol;         /* absolute residual tolerance of proj_mode 1, 2 */
   int proj_guess;          /* proj_mode 1, 2: 1 = start each solve from the previous substep's phi
                             * scaled by the ratio of the RK weights h_bar; 2 = from the guess of the
                             * network attached with ekm_set_warm_start_net (0 = from zero) */
   int proj_krylov;         /* proj_mode 1, 2: 1 = the outer iteration is GCR(1) (each cycle's
                             * correction made A-orthogonal to the previous one, then a minimal
-                            * residual step); 0 = plain iterative refinement */
+                            * residual step); 0 = plain iterative refinement.  It acts in V cycles
+                            * only: not in proj_mode 2 on a rectilinear grid, unless its separable
+                            * passes leave solves above proj_tol or its operator is not taken as
+                            * separable */
   int les_model;           /* LES_MODEL_TYPE of the velocity subgrid model (src/les_chan.F90):
                             * 0 = none (DNS), 2 = dynamic Smagorinsky */
   int sponge_type;         /* SPONGE_TYPE (input.dat, src/diablo.F90:278): 0 = none, 1 = parabolic,
@@ -127,7 +130,8 @@ typedef struct ekm_diag {
   int rk_step;          /* next RK_STEP to run (1..3) */
   int mg_solves;        /* real Poisson solves in the last projection */
   int mg_cycles;        /* W(2,1) cycles summed over those solves (reference iparm(17)); proj_mode 1, 2:
-                         * V(1,1) cycles and separable solves */
+                         * V(1,1) cycles and separable passes (from a zero start the first pass
+                         * runs before a residual is known, so a zero right-hand side counts one) */
   int mg_max_cycles;    /* largest cycle count of a single solve */
   int status;           /* status of the last substep */
   int mg_unconverged;   /* proj_mode 1/2: solves of the last projection that stopped at proj_maxit
