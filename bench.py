@@ -246,7 +246,7 @@ def main() -> int:
     ap.add_argument("--mode", type=int, default=2, help="headline projection form (0, 1, 2)")
     ap.add_argument("--tol", type=float, default=1e-12, help="max |residual| per real solve, modes 1 and 2")
     ap.add_argument("--krylov", type=int, default=1, choices=(0, 1),
-                    help="outer iteration of modes 1 and 2 (0: plain refinement, 1: GCR(1))")
+                    help="outer iteration of the V cycles (0: plain refinement, 1: GCR(1))")
     ap.add_argument("--side-steps", type=int, default=3, help="steps of the compared forms (0: skip them)")
     ap.add_argument("--side-warmup", type=int, default=4,
                     help="warm-up steps of the compared forms (4: the subgrid models' first refresh, at step 5, "

@@ -15,15 +15,16 @@
 //
 // with Ly = S^-1/2 Q Lambda Q' S^1/2 (a tridiagonal matrix with positive
 // products of its off-diagonals is similar to a symmetric one) and J = W(i) M(j).
-// One pass divides the residual by 1e4..1e5 for every kx alike (a V(1,1) cycle
-// by 20..1000), so the solves of a projection end together after 3 passes and
+// One pass divides the residual by 1e3 (33 rows) to 1e5 for every kx alike (a
+// V(1,1) cycle by 20..1000), so the solves of a projection end together after 3 passes and
 // none of them is a chain of one workgroup's memory round trips: 1024x385x769
 // is 684 solves of 4 to 8 V cycles otherwise.  A pass counts as one cycle.
 // Measured per projection against the V cycles: 1024x385x769 12.0 ms instead
 // of 68.8, 256x193x257 0.50 instead of 4.95.  Against a solve to 2e-14, a step
-// that stops at 1e-12 is 4 to 200 times closer in every field than with V cycles
-// (64x65x65 to 256x193x257, and a periodic singular set): the passes end further
-// below the tolerance, and leave less of the smooth error.
+// that stops at 1e-12 is 3 to 90 times closer in every field than with V cycles
+// (64x65x65 to 256x193x257, 32x129x385, and the reference run's periodic singular
+// set): the passes leave less of the smooth error, and end further below the
+// tolerance in most solves.
 //
 // The decomposition is tried at set-up (sep_plan_build) and used where every
 // coefficient lies within kSepDev of the separable operator's; what has not
@@ -42,8 +43,8 @@ namespace {
 // of both operators sum to zero without the kx^2 term, so a deviation acts on
 // differences of neighbours only and is not amplified on smooth modes: passes in
 // FP64 on sine, geometric, jumping and noisy spacings, 33 to 769 columns, every
-// kind of sides and kx = 0, reduce max|r| by 0.4 to 1.1 times the deviation each
-// (the first, by up to 14 times it).  0.02 keeps a pass at least as fast as the
+// kind of sides and kx = 0, reduce max|r| to at most 1.1 times the deviation each
+// (the first to at most 11 times it).  0.02 keeps a pass at least as fast as the
 // V(1,1) cycle's worst rate (about 1/20).
 constexpr double kSepDev = 0.02;
 // Lines whose shift lambda_k - kx^2 is below this fraction of the z operator's

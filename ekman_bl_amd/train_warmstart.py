@@ -5,7 +5,7 @@ gains (the learned warm-start study on the 256x193x257 stratified grid).
         [--heldout 10-12] [--steps 4] [--epochs 0] [--train-seconds 150]
 
 1. Pairs: for every training seed, one warm-up step of the headline form
-   (consistent projection, FP32 cycles, GCR(1), starts from zero), then
+   (consistent projection, FP32 solves, starts from zero), then
    `--steps` steps whose projections are dumped: each real solve's RHS_TMP,
    the previous projection's solution of the same solve, kx, and the
    converged solution (2 (NX/3+1) solves per projection).
