@@ -1,11 +1,11 @@
 // ekm_sep.hip -- separable solver of the consistent projection (proj_mode 2
 // on grids without cross terms; no counterpart in the reference).
 //
-// On a rectilinear grid the finest operator, row-scaled by 1/J, is to a few
-// 1e-5 the sum Lz + Ly - kx^2 of a tridiagonal operator in z and one in y
-// (the interior rows' metrics, the boundary rows of MUDPACK's discretisation
-// and J differ from the products of one-dimensional ones by that much).  The
-// separable operator is therefore solved directly in place of a V cycle, in
+// On a rectilinear grid the finest operator, row-scaled by 1/J, is to 1e-3 (33
+// rows) or 1e-5 (385 rows) the sum Lz + Ly - kx^2 of a tridiagonal operator in z
+// and one in y (the interior rows' metrics, the boundary rows of MUDPACK's
+// discretisation and J differ from the products of one-dimensional ones by that
+// much).  The separable operator is therefore solved directly in place of a V cycle, in
 // the cycle precision (FP32), inside the same FP64 residual iterations:
 //
 //   r^ = Q' S^1/2 M^-1 r            product over the rows j, one GEMM for all solves
@@ -16,15 +16,15 @@
 // with Ly = S^-1/2 Q Lambda Q' S^1/2 (a tridiagonal matrix with positive
 // products of its off-diagonals is similar to a symmetric one) and J = W(i) M(j).
 // One pass divides the residual by 1e3 (33 rows) to 1e5 for every kx alike (a
-// V(1,1) cycle by 20..1000), so the solves of a projection end together after 3 passes and
-// none of them is a chain of one workgroup's memory round trips: 1024x385x769
-// is 684 solves of 4 to 8 V cycles otherwise.  A pass counts as one cycle.
+// V(1,1) cycle by 20..1000), so the solves of a projection end together after 3
+// passes and none of them is a chain of one workgroup's memory round trips:
+// 1024x385x769 is 684 solves of 4 to 8 V cycles otherwise.  A pass counts as one cycle.
 // Measured per projection against the V cycles: 1024x385x769 12.0 ms instead
 // of 68.8, 256x193x257 0.50 instead of 4.95.  Against a solve to 2e-14, a step
 // that stops at 1e-12 is 3 to 90 times closer in every field than with V cycles
-// (64x65x65 to 256x193x257, 32x129x385, and the reference run's periodic singular
-// set): the passes leave less of the smooth error, and end further below the
-// tolerance in most solves.
+// (planes of 65x65 to 385x769, and the reference run's periodic singular set): the
+// passes leave less of the smooth error, and end further below the tolerance in
+// most solves.
 //
 // The decomposition is tried at set-up (sep_plan_build) and used where every
 // coefficient lies within kSepDev of the separable operator's; what has not
